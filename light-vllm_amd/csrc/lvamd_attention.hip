@@ -4,6 +4,8 @@
 
 #include "lvamd_common.h"
 
+using namespace lvamd;
+
 extern "C" int lvamd_paged_attention(const lvamd_attention_plan* plan,
                                      const void* q, int64_t q_token_stride, int64_t q_head_stride,
                                      const void* new_key, int64_t new_key_token_stride,
@@ -24,9 +26,9 @@ extern "C" int lvamd_paged_attention(const lvamd_attention_plan* plan,
                                 p.col_tiles, p.group_waves, p.block_size, scale, p.dtype, stream);
     if (status != LVAMD_OK) return status;
     if (p.num_jobs > 0) {
-      status = lvamd_paged_attention_merge(p.part_acc, p.part_ml, out, out_token_stride, out_head_stride, p.jobs,
-                                           p.num_jobs, p.num_kv_heads, p.group, p.head_size, p.col_tiles,
-                                           p.merge_columns, p.dtype, stream);
+      status = launch_merge(p.part_acc, p.part_ml, out, out_token_stride, out_head_stride, p.jobs, p.num_jobs,
+                            p.num_partial_slots, p.num_kv_heads, p.group, p.head_size, p.col_tiles, p.merge_columns,
+                            p.dtype, static_cast<hipStream_t>(stream));
       if (status != LVAMD_OK) return status;
     }
   }
@@ -39,10 +41,10 @@ extern "C" int lvamd_paged_attention(const lvamd_attention_plan* plan,
                                  p.block_size, scale, p.dtype, stream);
     if (status != LVAMD_OK) return status;
     if (p.num_prefill_jobs > 0) {
-      status = lvamd_paged_attention_merge(p.prefill_part_acc, p.prefill_part_ml, out, out_token_stride,
-                                           out_head_stride, p.prefill_jobs, p.num_prefill_jobs, p.num_kv_heads,
-                                           p.group, p.head_size, p.prefill_col_tiles, p.prefill_merge_columns,
-                                           p.dtype, stream);
+      status = launch_merge(p.prefill_part_acc, p.prefill_part_ml, out, out_token_stride, out_head_stride,
+                            p.prefill_jobs, p.num_prefill_jobs, p.num_prefill_partial_slots, p.num_kv_heads, p.group,
+                            p.head_size, p.prefill_col_tiles, p.prefill_merge_columns, p.dtype,
+                            static_cast<hipStream_t>(stream));
     }
   }
   return status;

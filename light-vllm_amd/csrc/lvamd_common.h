@@ -89,21 +89,6 @@ __device__ __forceinline__ void store_partial4(T* p, f32x4 v, float s) {
 
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 
-// N consecutive partial elements (N = 1, 2 or 4): one load, converted to
-// fp32 apart from it (partial_f32) so that a caller can issue all its loads
-// before the first conversion waits.
-template <typename T, int N> struct PartialVec { typedef T type __attribute__((ext_vector_type(N))); };
-template <typename T> struct PartialVec<T, 1> { typedef T type; };
-
-template <typename T, int N>
-__device__ __forceinline__ float partial_f32(const typename PartialVec<T, N>::type& x, int k) {
-  if constexpr (N == 1) {
-    return to_f32(x);
-  } else {
-    return to_f32<T>(x[k]);
-  }
-}
-
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
 typedef short s16x4 __attribute__((ext_vector_type(4)));
@@ -172,5 +157,12 @@ inline int dtype_size(int dtype) {
 inline int launch_status() {
   return hipGetLastError() == hipSuccess ? LVAMD_OK : LVAMD_ERR_LAUNCH;
 }
+
+// lvamd_paged_attention_merge with the launch's partial count (all jobs; 0:
+// unknown), which picks the kernel's shape.
+int launch_merge(const void* part_acc, const float* part_ml, void* out, int64_t out_token_stride,
+                 int64_t out_head_stride, const int32_t* jobs, int32_t num_jobs, int64_t num_partials,
+                 int32_t num_kv_heads, int32_t group, int32_t head_size, int32_t col_tiles, int32_t max_columns,
+                 int32_t dtype, hipStream_t s);
 
 }  // namespace lvamd

@@ -902,13 +902,24 @@ __global__ __launch_bounds__(64 * WG) void paged_decode_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// Merge: one wave per (job, kv head, column); a workgroup holds the four
-// waves of four consecutive columns.  Lane l combines dims EPL*l..+EPL-1 of
-// its column over the job's partials, MCP partials per round trip (their
-// (max, sum) pairs and normalised rows are all requested before any is
-// used), by log-sum-exp in the log2 domain: partial i weighs
-// sum_i * 2^(max_i - max).  Every lane computes the chunk's weights itself
-// from the same (max, sum) values, so no cross-lane step is needed.
+// Merge: combines each output column's partials by log-sum-exp in the log2
+// domain: partial i weighs sum_i * 2^(max_i - max).  A lane holds one 16-byte
+// chunk of a column's row, so a wave works on 64 / (chunks per row) columns at
+// once (four at D = 128 in 16 bits) and requests up to MCP partials of each
+// (their (max, sum) pairs and normalised rows) before it uses any; every
+// lane computes its column's weights itself from the same pairs, so no
+// cross-lane step is needed.
+//
+// A merge is two dependent memory round trips (job record, partials) when
+// its columns are few, and bound by the partials' bytes when they are many.
+// P = 1: a workgroup's four waves take four sets of columns.  P = 4 and 16:
+// its P waves take the same columns and every P-th partial each, and the
+// first wave adds their results up from LDS, so that a job of many partials
+// is still one round trip.  Measured on MI355X against one column per wave
+// with loads of one to four elements per lane (the earlier form): 57,344
+// columns of two partials (a 2,048-token chunk, D = 128 bf16) 29.6 -> 12.5 us,
+// 1.9 TB/s -> 4.4 TB/s; 896 columns of about 15 (64 sequences, D = 64 fp16)
+// 6.4 -> 4.8 us; 28 columns of 44 (one sequence of 8K) 6.1 -> 4.5 us.
 // ---------------------------------------------------------------------------
 // The fields a wave needs first (its job record's address) are scalar kernel
 // arguments ahead of the rest: the build preloads leading scalar arguments
@@ -921,34 +932,47 @@ struct MergeArgs {
   int64_t out_tok_stride, out_head_stride;
 };
 
-constexpr int kMergeWaves = 4;  // columns (waves) per merge workgroup
+constexpr int kMergeRoundTrip = 16;  // partials a wave requests at once
+constexpr int merge_waves(int p) { return p == 1 ? 4 : p; }  // waves per workgroup
 
 template <typename T, int D>
-__global__ __launch_bounds__(64 * kMergeWaves) void paged_merge_kernel(
+struct MergeShape {
+  static constexpr int EPC = 16 / (int)sizeof(T);  // elements per lane
+  static constexpr int CPR = D / EPC;              // chunks per row
+  static constexpr int LPC = CPR <= 4 ? 4 : CPR <= 8 ? 8 : CPR <= 16 ? 16 : CPR <= 32 ? 32 : 64;  // lanes per column
+  static constexpr int CW = 64 / LPC;              // columns per wave
+};
+template <typename T, int D, int P>
+constexpr int merge_columns = MergeShape<T, D>::CW * (merge_waves(P) / P);  // per workgroup
+
+template <typename T, int D, int P>
+__global__ __launch_bounds__(64 * merge_waves(P)) void paged_merge_kernel(
     const int32_t* __restrict__ jobs,  // [num_jobs][LVAMD_MERGE_FIELDS]
-    const int32_t quads,               // workgroups (of kMergeWaves columns) per (job, kv head)
+    const int32_t groups,              // workgroups (of merge_columns columns) per (job, kv head)
     const int32_t num_kv_heads, const int32_t group,
     const int32_t col_tiles,           // column tiles per partial slot (the decode launch's)
     const MergeArgs a) {
-  constexpr int EPL = D <= 64 ? 1 : (D <= 128 ? 2 : 4);  // dims per lane
-  constexpr int MCP = 16;
+  using S = MergeShape<T, D>;
+  constexpr int EPC = S::EPC, MCP = kMergeRoundTrip;
   const int Hkv = num_kv_heads;
   const int G = group;
   const int cols = 16 * col_tiles;  // columns per partial slot
-  const int jh = (int)blockIdx.x / quads;
-  const int c = ((int)blockIdx.x - jh * quads) * kMergeWaves +
-                __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int lane = threadIdx.x & 63;
+  const int jh = (int)blockIdx.x / groups;
+  const int c0 = ((int)blockIdx.x - jh * groups) * merge_columns<T, D, P> + (P == 1 ? wave * S::CW : 0);
   const int job = jh / Hkv;
   const int kvh = jh - job * Hkv;
-  const int lane = threadIdx.x & 63;
   const int32_t* jb = jobs + (int64_t)job * LVAMD_MERGE_FIELDS;
   const int cgroup = jb[1], slot0 = jb[2], np = jb[3], q_start = jb[4], q_len = jb[5];
-  const int col = cgroup * cols + c;
-  if (col >= q_len * G) return;
+  const int col_end = min(cols, q_len * G - cgroup * cols);  // the slot's columns in use
+  if (c0 >= col_end) return;  // (P > 1: the whole workgroup's)
+  const int ch = lane & (S::LPC - 1);
+  const int c = c0 + lane / S::LPC;
+  const bool act = c < col_end && ch < S::CPR;
+  const int col = cgroup * cols + (c < col_end ? c : c0);
   const int qi = col / G;
   const int qhead = kvh * G + (col - qi * G);
-  const int e0 = lane * EPL;
-  const bool act = e0 < D;
   // A request whose shared prefix was attended by span units (prefill jobs
   // only): fields 6 = first span partial slot + 1, 7 = the request's first
   // column within the span | pieces per span unit << 24.  Column v of the
@@ -960,40 +984,36 @@ __global__ __launch_bounds__(64 * kMergeWaves) void paged_merge_kernel(
   const int sunit = sv / cols;
   const int scol = sv - sunit * cols;
   const int ntot = np + span_pieces;
+  // Partial rows of this column: its own pieces, then its span unit's.
+  const int64_t row_step = (int64_t)Hkv * cols;
+  const int64_t own = ((int64_t)slot0 * Hkv + kvh) * cols + c;
+  const int64_t shared = ((int64_t)(span_slot + sunit * span_pieces - np) * Hkv + kvh) * cols + scol;
 
   float mrun = -INFINITY;
   float lsum = 0.f;
-  float o[EPL];
+  float o[EPC];
 #pragma unroll
-  for (int k = 0; k < EPL; ++k) o[k] = 0.f;
-  for (int p0 = 0; p0 < ntot; p0 += MCP) {
-    const int n = ntot - p0 < MCP ? ntot - p0 : MCP;
-    typedef typename PartialVec<T, EPL>::type Raw;
+  for (int k = 0; k < EPC; ++k) o[k] = 0.f;
+  // Wave w of P > 1 takes partials w, w + P, ...
+  for (int p0 = P == 1 ? 0 : wave; p0 < ntot; p0 += MCP * P) {
+    const int n = (ntot - p0 + P - 1) / P;  // partials left (more than MCP: another round)
     float2 ml[MCP];
-    Raw raw[MCP];
+    u32x4 raw[MCP];
     // Entries past the job load nothing and carry max -inf (weight 0).  No
     // loaded value is used before the barrier, so the round trip's loads all
-    // issue before the first wait: the (max, sum) pairs are scalar loads,
-    // and a use scheduled between them (a 16-bit row's conversion) waits for
-    // every one issued so far.
+    // issue before the first wait.
 #pragma unroll
     for (int i = 0; i < MCP; ++i) {
       ml[i] = make_float2(-INFINITY, 0.f);
-      raw[i] = Raw{};
-      if (i < n) {
-        const int p = p0 + i;
-        const int64_t r = p < np ? ((int64_t)(slot0 + p) * Hkv + kvh) * cols + c
-                                 : ((int64_t)(span_slot + sunit * span_pieces + (p - np)) * Hkv + kvh) * cols + scol;
+      raw[i] = u32x4{0u, 0u, 0u, 0u};
+      if (i < n && act) {
+        const int p = p0 + i * P;
+        const int64_t r = (p < np ? own : shared) + p * row_step;
         ml[i] = *reinterpret_cast<const float2*>(a.part_ml + r * 2);
-        if (act) raw[i] = *reinterpret_cast<const Raw*>(static_cast<const T*>(a.part_acc) + r * D + e0);
+        raw[i] = *reinterpret_cast<const u32x4*>(static_cast<const T*>(a.part_acc) + r * D + ch * EPC);
       }
     }
     __builtin_amdgcn_sched_barrier(0);
-    float pa[MCP][EPL];
-#pragma unroll
-    for (int i = 0; i < MCP; ++i)
-#pragma unroll
-      for (int k = 0; k < EPL; ++k) pa[i][k] = partial_f32<T, EPL>(raw[i], k);
     float mc = -INFINITY;
 #pragma unroll
     for (int i = 0; i < MCP; ++i) mc = fmaxf(mc, ml[i].x);
@@ -1002,22 +1022,53 @@ __global__ __launch_bounds__(64 * kMergeWaves) void paged_merge_kernel(
     const float sc = (any && mrun != -INFINITY) ? fast_exp2(mrun - mnew) : (any ? 0.f : 1.f);
     lsum *= sc;
 #pragma unroll
-    for (int k = 0; k < EPL; ++k) o[k] *= sc;
+    for (int k = 0; k < EPC; ++k) o[k] *= sc;
 #pragma unroll
     for (int i = 0; i < MCP; ++i) {
-      // Entries past the job and empty partials carry max -inf: weight 0.
-      const float wt = ml[i].x != -INFINITY ? fast_exp2(ml[i].x - mnew) * ml[i].y : 0.f;
-      lsum += wt;
+      if (i < n) {  // (uniform: short jobs skip the rest)
+        // Empty partials carry max -inf: weight 0.
+        const float wt = ml[i].x != -INFINITY ? fast_exp2(ml[i].x - mnew) * ml[i].y : 0.f;
+        lsum += wt;
+        T row[EPC];
+        __builtin_memcpy(row, &raw[i], 16);
 #pragma unroll
-      for (int k = 0; k < EPL; ++k) o[k] += wt * pa[i][k];
+        for (int k = 0; k < EPC; ++k) o[k] += wt * to_f32(row[k]);
+      }
     }
     mrun = mnew;
+  }
+  if constexpr (P > 1) {
+    // The other waves' (max, sum) and rows through LDS to the first wave.
+    __shared__ float part[P - 1][2 + EPC][64];
+    if (wave > 0) {
+      part[wave - 1][0][lane] = mrun;
+      part[wave - 1][1][lane] = lsum;
+#pragma unroll
+      for (int k = 0; k < EPC; ++k) part[wave - 1][2 + k][lane] = o[k];
+    }
+    __syncthreads();
+    if (wave > 0) return;
+    float m = mrun;
+#pragma unroll
+    for (int w = 0; w < P - 1; ++w) m = fmaxf(m, part[w][0][lane]);
+    const float own_w = mrun != -INFINITY ? fast_exp2(mrun - m) : 0.f;
+    lsum *= own_w;
+#pragma unroll
+    for (int k = 0; k < EPC; ++k) o[k] *= own_w;
+#pragma unroll
+    for (int w = 0; w < P - 1; ++w) {
+      const float mw = part[w][0][lane];
+      const float wt = mw != -INFINITY ? fast_exp2(mw - m) : 0.f;
+      lsum += wt * part[w][1][lane];
+#pragma unroll
+      for (int k = 0; k < EPC; ++k) o[k] += wt * part[w][2 + k][lane];
+    }
   }
   if (!act) return;
   const float inv = lsum > 0.f ? 1.f / lsum : 0.f;
   T* orow = static_cast<T*>(a.out) + (int64_t)(q_start + qi) * a.out_tok_stride + (int64_t)qhead * a.out_head_stride;
 #pragma unroll
-  for (int k = 0; k < EPL; ++k) orow[e0 + k] = from_f32<T>(o[k] * inv);
+  for (int k = 0; k < EPC; ++k) orow[ch * EPC + k] = from_f32<T>(o[k] * inv);
 }
 
 // ---------------------------------------------------------------------------
@@ -1084,29 +1135,46 @@ static int dispatch_decode(int dtype, int head_size, int col_tiles, F f) {
   }
 }
 
-template <typename T>
-static int launch_merge_t(int head_size, dim3 grid, hipStream_t s, const int32_t* jobs, int32_t quads,
+// One workgroup per (job, kv head, merge_columns columns), over the columns
+// the jobs use; columns past a job's own count exit at once.
+template <typename T, int D, int P>
+static int launch_merge_p(int64_t job_heads, int64_t max_columns, hipStream_t s, const int32_t* jobs,
                           int32_t num_kv_heads, int32_t group, int32_t col_tiles, const MergeArgs& a) {
-  const dim3 block(64 * kMergeWaves);
-  switch (head_size) {
-    case 32: hipLaunchKernelGGL((paged_merge_kernel<T, 32>), grid, block, 0, s, jobs, quads, num_kv_heads, group, col_tiles, a); break;
-    case 48: hipLaunchKernelGGL((paged_merge_kernel<T, 48>), grid, block, 0, s, jobs, quads, num_kv_heads, group, col_tiles, a); break;
-    case 64: hipLaunchKernelGGL((paged_merge_kernel<T, 64>), grid, block, 0, s, jobs, quads, num_kv_heads, group, col_tiles, a); break;
-    case 80: hipLaunchKernelGGL((paged_merge_kernel<T, 80>), grid, block, 0, s, jobs, quads, num_kv_heads, group, col_tiles, a); break;
-    case 96: hipLaunchKernelGGL((paged_merge_kernel<T, 96>), grid, block, 0, s, jobs, quads, num_kv_heads, group, col_tiles, a); break;
-    case 112: hipLaunchKernelGGL((paged_merge_kernel<T, 112>), grid, block, 0, s, jobs, quads, num_kv_heads, group, col_tiles, a); break;
-    case 128: hipLaunchKernelGGL((paged_merge_kernel<T, 128>), grid, block, 0, s, jobs, quads, num_kv_heads, group, col_tiles, a); break;
-    case 144: hipLaunchKernelGGL((paged_merge_kernel<T, 144>), grid, block, 0, s, jobs, quads, num_kv_heads, group, col_tiles, a); break;
-    case 160: hipLaunchKernelGGL((paged_merge_kernel<T, 160>), grid, block, 0, s, jobs, quads, num_kv_heads, group, col_tiles, a); break;
-    case 176: hipLaunchKernelGGL((paged_merge_kernel<T, 176>), grid, block, 0, s, jobs, quads, num_kv_heads, group, col_tiles, a); break;
-    case 192: hipLaunchKernelGGL((paged_merge_kernel<T, 192>), grid, block, 0, s, jobs, quads, num_kv_heads, group, col_tiles, a); break;
-    case 208: hipLaunchKernelGGL((paged_merge_kernel<T, 208>), grid, block, 0, s, jobs, quads, num_kv_heads, group, col_tiles, a); break;
-    case 224: hipLaunchKernelGGL((paged_merge_kernel<T, 224>), grid, block, 0, s, jobs, quads, num_kv_heads, group, col_tiles, a); break;
-    case 240: hipLaunchKernelGGL((paged_merge_kernel<T, 240>), grid, block, 0, s, jobs, quads, num_kv_heads, group, col_tiles, a); break;
-    case 256: hipLaunchKernelGGL((paged_merge_kernel<T, 256>), grid, block, 0, s, jobs, quads, num_kv_heads, group, col_tiles, a); break;
-    default: return LVAMD_ERR_UNSUPPORTED;
-  }
+  const int64_t groups = (max_columns + merge_columns<T, D, P> - 1) / merge_columns<T, D, P>;
+  if (job_heads * groups > 0x7fffffffLL) return LVAMD_ERR_INVALID_ARGUMENT;
+  hipLaunchKernelGGL((paged_merge_kernel<T, D, P>), dim3((unsigned)(job_heads * groups)), dim3(64 * merge_waves(P)), 0,
+                     s, jobs, (int32_t)groups, num_kv_heads, group, col_tiles, a);
   return launch_status();
+}
+
+int launch_merge(const void* part_acc, const float* part_ml, void* out, int64_t out_token_stride,
+                 int64_t out_head_stride, const int32_t* jobs, int32_t num_jobs, int64_t num_partials,
+                 int32_t num_kv_heads, int32_t group, int32_t head_size, int32_t col_tiles, int32_t max_columns,
+                 int32_t dtype, hipStream_t s) {
+  if (dtype_size(dtype) == 0 || !head_size_supported(head_size) || col_tiles < 1 || col_tiles > 16)
+    return LVAMD_ERR_UNSUPPORTED;
+  if (max_columns < 1 || max_columns > 16 * col_tiles) return LVAMD_ERR_INVALID_ARGUMENT;
+  if (num_jobs < 0 || num_kv_heads <= 0 || group <= 0) return LVAMD_ERR_INVALID_ARGUMENT;
+  if (num_jobs == 0) return LVAMD_OK;
+  if (!part_acc || !part_ml || !out || !jobs) return LVAMD_ERR_INVALID_ARGUMENT;
+  MergeArgs a;
+  a.part_acc = part_acc;
+  a.part_ml = part_ml;
+  a.out = out;
+  a.out_tok_stride = out_token_stride;
+  a.out_head_stride = out_head_stride;
+  const int64_t job_heads = (int64_t)num_jobs * num_kv_heads;
+  return dispatch_decode(dtype, head_size, 1, [&]<typename T, int D, int CTW>() -> int {
+    // Partials per job on average: one wave's requests grow with them (192
+    // columns of 13: 4.6 us at P = 1, 4.1 at P = 4; 1,792 columns of five:
+    // the same at both), and 129 partials take P = 4 three round trips
+    // (6.2 us against 4.6 at P = 16).
+    if (num_partials > 32 * (int64_t)num_jobs)
+      return launch_merge_p<T, D, 16>(job_heads, max_columns, s, jobs, num_kv_heads, group, col_tiles, a);
+    if (num_partials > 8 * (int64_t)num_jobs)
+      return launch_merge_p<T, D, 4>(job_heads, max_columns, s, jobs, num_kv_heads, group, col_tiles, a);
+    return launch_merge_p<T, D, 1>(job_heads, max_columns, s, jobs, num_kv_heads, group, col_tiles, a);
+  });
 }
 
 }  // namespace lvamd
@@ -1236,28 +1304,6 @@ extern "C" int lvamd_paged_attention_merge(const void* part_acc, const float* pa
                                            const int32_t* jobs, int32_t num_jobs,
                                            int32_t num_kv_heads, int32_t group, int32_t head_size, int32_t col_tiles,
                                            int32_t max_columns, int32_t dtype, lvamd_stream_t stream) {
-  if (dtype_size(dtype) == 0 || !head_size_supported(head_size) || col_tiles < 1 || col_tiles > 16)
-    return LVAMD_ERR_UNSUPPORTED;
-  if (max_columns < 1 || max_columns > 16 * col_tiles) return LVAMD_ERR_INVALID_ARGUMENT;
-  if (num_jobs < 0 || num_kv_heads <= 0 || group <= 0) return LVAMD_ERR_INVALID_ARGUMENT;
-  if (num_jobs == 0) return LVAMD_OK;
-  if (!part_acc || !part_ml || !out || !jobs) return LVAMD_ERR_INVALID_ARGUMENT;
-  const int64_t quads = (max_columns + kMergeWaves - 1) / kMergeWaves;
-  if ((int64_t)num_jobs * num_kv_heads * quads > 0x7fffffffLL) return LVAMD_ERR_INVALID_ARGUMENT;
-  MergeArgs a;
-  a.part_acc = part_acc;
-  a.part_ml = part_ml;
-  a.out = out;
-  a.out_tok_stride = out_token_stride;
-  a.out_head_stride = out_head_stride;
-  // One workgroup per (job, kv head, kMergeWaves columns), over the columns
-  // the jobs use; columns past a job's own count exit at once.
-  const dim3 grid((unsigned)(num_jobs * num_kv_heads * quads));
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  const int32_t q = (int32_t)quads;
-  switch (dtype) {
-    case LVAMD_BF16: return launch_merge_t<__bf16>(head_size, grid, s, jobs, q, num_kv_heads, group, col_tiles, a);
-    case LVAMD_F16: return launch_merge_t<_Float16>(head_size, grid, s, jobs, q, num_kv_heads, group, col_tiles, a);
-    default: return launch_merge_t<float>(head_size, grid, s, jobs, q, num_kv_heads, group, col_tiles, a);
-  }
+  return launch_merge(part_acc, part_ml, out, out_token_stride, out_head_stride, jobs, num_jobs, 0, num_kv_heads,
+                      group, head_size, col_tiles, max_columns, dtype, static_cast<hipStream_t>(stream));
 }
