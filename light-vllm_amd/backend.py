@@ -35,7 +35,8 @@ from light_vllm_amd import errors, native
 from light_vllm_amd.metadata import PagedAttentionMetadata
 from light_vllm_amd.paged_cache import current_stream, dtype_code, hip_append_rotary
 from light_vllm_amd.plan import (
-    DECODE_MAX_COLUMNS, DECODE_MIN_UNITS_PER_WAVE, PREFILL_MIN_TILES, UNIT_TOKENS, LayerShapes, Staging, StepPlan,
+    DECODE_MAX_COLUMNS, DECODE_MERGE_PIECES, DECODE_MIN_UNITS_PER_WAVE, PREFILL_MIN_TILES, UNIT_TOKENS, LayerShapes,
+    Staging, StepPlan,
 )
 
 # Head sizes the kernels are built for: multiples of 16 from 32 to 256.
@@ -542,7 +543,7 @@ class HipPagedAttentionBackend:
                 int(self._shared_prefix),
                 native.xcd_count() if columns else 0, self._prefill_order,
                 native.decode_split_groups(code, d) if self._decode_workgroups else 0,
-                native.decode_split_waves(code, d),
+                native.decode_split_waves(code, d), DECODE_MERGE_PIECES,
             )
             self._facts[key] = found
         return found

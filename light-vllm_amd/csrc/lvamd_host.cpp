@@ -949,6 +949,7 @@ struct DecodeParams {
   int64_t group, col_tiles, max_cols, hkv, resident, bs, min_units, max_units, unit;
   int64_t split_groups = 0;  // resident workgroups of the workgroup-split kernel (0: not built)
   int64_t split_waves = 0;   // its waves per workgroup
+  int64_t merge_pieces = 0;  // most pieces of a segment the merge takes well (0: kMergePiecesMax)
 };
 
 // Workgroup split of the decode kernel: workgroups of split_waves waves, one
@@ -975,6 +976,14 @@ struct DecodeParams {
 // host time per layer on the split, 313 us and 9.3 us on stream-K).)
 constexpr int64_t kSplitMergeTiles = 3;
 constexpr int64_t kMergePiecesMax = 48;
+// With the merge's sixteen-wave shape (merge_pieces above kMergePiecesMax) a
+// lone long sequence is spread over up to that many shares: one tile each up
+// to kOneTilePieces of them, two or more past that.  Per layer at 28 / 4
+// heads, D 128, bf16: one sequence of 8,112 tokens (254 tiles) 23.3 us in 43
+// shares of six tiles, 17.9 in 86 of three, 16.9 in 127 of two, 19.4 in 254
+// of one; 32,701 tokens 58 us in 47 shares, 32.4 in 147, 30.6 in 205; 2,048
+// tokens 13.2 us in 33 shares of two, 12.8 in 64 of one.
+constexpr int64_t kOneTilePieces = 96;
 constexpr int64_t kSplitMaxTiles = 2;
 constexpr int64_t kSplitBusyGroups = 128;
 
@@ -999,14 +1008,13 @@ void build_decode(const Requests& q, const int32_t* ids, int64_t nflat, const De
   int64_t cap = std::max<int64_t>(1, ((kTableSlice - 2) * d.bs) / d.unit);
   if (d.max_units > 0) cap = std::max<int64_t>(1, std::min(cap, d.max_units));
   // Shares of at least min_units tiles, and long enough that no segment is
-  // cut into more than kMergePiecesMax pieces (a segment of T tiles over
-  // shares of P takes at most ceil(T / P) + 1; the merge reads 16 partials
-  // per round trip: one sequence of 2048 tokens in 65 one-tile pieces took
-  // 15.7 us per layer against 14.9 in 33).
+  // cut into more pieces than the merge takes well (a segment of T tiles over
+  // shares of P takes at most ceil(T / P) + 1).
+  const int64_t most = d.merge_pieces > 1 ? d.merge_pieces : kMergePiecesMax;
   int64_t longest_seg = 0;
   for (const Seg& sg : segs) longest_seg = std::max(longest_seg, sg.tiles);
-  const int64_t min_units =
-      std::max<int64_t>(d.min_units, (longest_seg + kMergePiecesMax - 2) / (kMergePiecesMax - 1));
+  int64_t min_units = std::max<int64_t>(d.min_units, (longest_seg + most - 2) / (most - 1));
+  if (most > kOneTilePieces && longest_seg > kOneTilePieces) min_units = std::max<int64_t>(min_units, 2);
   int64_t waves = std::max<int64_t>(
       1, std::min(std::max<int64_t>(1, d.resident / d.hkv), (total + min_units - 1) / min_units));
   waves = std::max(waves, (total + cap - 1) / cap);
@@ -1627,7 +1635,7 @@ PyObject* prefill_work(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   return prefill_result(out);
 }
 
-// layer_work(req_meta i32[B*8], flat i32, kernel facts (int64 array, 23
+// layer_work(req_meta i32[B*8], flat i32, kernel facts (int64 array, 26
 //            entries, below), cost4, wide_max_tiles)
 //   -> (col_tiles, prefill_waves, decode result or None, prefill result or None)
 //
@@ -1645,8 +1653,8 @@ PyObject* prefill_work(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
 //   (0: no per-XCD order of the prefill grid), 22 per-XCD order (0: grouped
 //   when its simulated packing is no slower, 1: grouped, 2: plain), 23
 //   resident workgroups of the workgroup-split decode kernel (0: never), 24
-//   its waves per workgroup.
-constexpr int kKernelFacts = 25;
+//   its waves per workgroup, 25 most decode pieces of a segment (0: 48).
+constexpr int kKernelFacts = 26;
 
 // One layer shape's plan: the choices and the lists of both kernels.
 struct LayerPlan {
@@ -1735,7 +1743,7 @@ const char* plan_layer(const Requests& q, const int32_t* ids, int64_t nflat, con
     const int64_t unit = ctw == 4 ? k[13] : k[11];
     const int64_t max_units = (k[16] > 0 && unit > 0) ? std::max<int64_t>(1, k[16] / unit) : 0;
     DecodeParams d{group, ctw, max_cols, hkv, ctw == 4 ? k[12] : k[10], bs, k[18] > 0 ? k[18] : 4, max_units, unit,
-                   k[23], k[24]};
+                   k[23], k[24], k[25]};
     if (d.unit <= 0 || d.resident <= 0) return "missing decode kernel facts";
     build_decode(q, ids, nflat, d, out.dec);
     out.has_dec = true;
@@ -1750,7 +1758,7 @@ const char* plan_layer(const Requests& q, const int32_t* ids, int64_t nflat, con
 // ---------------------------------------------------------------------------
 // plan_step(flat i32, counts i64, computed i64, reserved i64, readonly i64,
 //           q_lens i64, vis_off i64, vis_words i64, vis u32, num_blocks,
-//           block_size, kernel facts i64 [n][25], cost4, wide_max_tiles,
+//           block_size, kernel facts i64 [n][26], cost4, wide_max_tiles,
 //           out i32 (writable))
 //   -> rule (int 1..6): a block-table rule fails (validate's codes);
 //      (needed, None, None): ``out`` holds fewer than ``needed`` entries;

@@ -46,6 +46,9 @@ DECODE_MAX_COLUMNS = 16
 # longer set the step's pace); steps that fill the resident waves are not
 # affected.
 DECODE_MIN_UNITS_PER_WAVE = 1
+# Most pieces of one decode segment: the merge's sixteen-wave shape combines
+# 256 partials in one round trip.
+DECODE_MERGE_PIECES = 256
 # Smallest key range (in prefill key tiles) the planner gives one prefill
 # workgroup when it splits units to fill the GPU.
 PREFILL_MIN_TILES = 4
@@ -542,7 +545,7 @@ class StepPlan:
         found = self._work.get(kernel_facts)
         if found is None:
             ctw, waves, dec, pre = native.host().layer_work(
-                self._req_meta, self.facts.raw[0], np.asarray(kernel_facts, dtype=np.int64), COL_TILES4_COST,
+                self._req_meta, self.facts.raw[0], np.asarray(_full_facts(kernel_facts), dtype=np.int64), COL_TILES4_COST,
                 float(PREFILL_WIDE_MAX_TILES),
             )
             found = DecodeWork(col_tiles=int(ctw), prefill_waves=int(waves))
@@ -594,8 +597,20 @@ KERNEL_FACTS = (
     "resident_waves_1", "tile_tokens_1", "resident_waves_4", "tile_tokens_4",
     "prefill_resident_4", "prefill_resident_8", "partition_tokens", "decode_max_columns",
     "min_units_per_wave", "prefill_min_tiles", "shared_prefix", "xcds", "prefill_order", "split_groups",
-    "split_waves",
+    "split_waves", "decode_merge_pieces",
 )
+# Facts that a row may leave out, with their values (0: the planner's own).
+_OPTIONAL_FACTS = (0,)
+
+
+def _full_facts(row) -> tuple[int, ...]:
+    """A kernel-facts row with its optional trailing facts filled in."""
+
+    row = tuple(int(v) for v in row)
+    missing = len(KERNEL_FACTS) - len(row)
+    if not 0 <= missing <= len(_OPTIONAL_FACTS):
+        raise ValueError(f"each layer shape needs {len(KERNEL_FACTS)} kernel facts")
+    return row + _OPTIONAL_FACTS[len(_OPTIONAL_FACTS) - missing:]
 
 
 class LayerShapes:
@@ -606,9 +621,7 @@ class LayerShapes:
     __slots__ = ("keys", "array")
 
     def __init__(self, rows) -> None:
-        self.keys = tuple(tuple(int(v) for v in row) for row in rows)
-        if any(len(row) != len(KERNEL_FACTS) for row in self.keys):
-            raise ValueError(f"each layer shape needs {len(KERNEL_FACTS)} kernel facts")
+        self.keys = tuple(_full_facts(row) for row in rows)
         self.array = np.asarray(self.keys, dtype=np.int64).reshape(-1)
 
 
