@@ -12,11 +12,13 @@
 //     (query, head-in-group) pair of one kv head, so the GQA group shares
 //     every K/V byte.  One workgroup per (unit, kv head): four waves of two
 //     16-column tiles, or eight waves of one (the host picks per step).
-//   * Keys go in 64-token tiles (32 for D = 256).  Each lane copies one
+//   * Keys go in 64-token tiles (32 above D = 128).  Each lane copies one
 //     16-byte chunk of one row per load straight from the pool (or this
 //     step's K/V) into LDS (global_load_lds_dwordx4: no registers, no LDS
 //     store instructions), double-buffered, one barrier per tile: tile t+1
 //     lands while tile t computes, tile t+2's table entries are in flight.
+//     With blocks of 16 tokens or more the 16 rows that a wave loads lie in
+//     one block, so their addresses are scalar (the B16 kernels).
 //     The LDS layout is unpadded and XOR-swizzled (below) so that the
 //     loads, the K reads and the V transpose reads are all free of bank
 //     conflicts.
@@ -30,7 +32,7 @@
 //     from the matrix cores (a ones row times P^T).
 //   * The append is fused: keys of this step's tokens are read from the
 //     step's K/V, and the unit that holds a token's own query writes its row
-//     to the pool.
+//     to the pool, out of the LDS tile.
 //   * A record with zero columns is padding of the planner's per-XCD order.
 //   * Split-K: a unit may cover a key range of its request (a piece); a piece
 //     that is not the whole range writes partials (its normalised output
@@ -42,6 +44,7 @@
 #include <type_traits>
 
 #include "lvamd_common.h"
+
 
 namespace lvamd {
 
@@ -58,14 +61,25 @@ constexpr int kPrefillKeyTile = 64;
 //   up to 256 registers per wave, two waves per SIMD (two workgroups per CU).
 // * W = 8 waves of one column tile: half the registers (128), four waves per
 //   SIMD to hide the softmax's dependency chain, twice the LDS reads per MFMA.
-// W = 8 is faster on split-K and short units (tree verification, chunks
-// without history), W = 4 on long unsplit units.  Keys per LDS tile: 64 (32
-// for D = 256, which is built for W = 4 only).
+// W = 8 is faster where a workgroup has few key tiles (tree verification,
+// short prompts), W = 4 elsewhere; the planner's rule holds the figures.  Keys
+// per LDS tile: 64 (32 above D = 128, built for W = 4 only).
+//
+// What bounds it (a 2,048-token chunk over 14K of history, D = 128 bf16, 28 / 4
+// heads, W = 4): the card runs the launch at 1.85-2.0 GHz (power), the matrix
+// cores are busy 47% of the cycles at 1.58 waves per SIMD on average, and in
+// timing-only copies neither the exponentials (-4%), the LDS reads (half of
+// them: -4%) nor the tile loads (none: -14%) alone are the bound.  468 us per
+// layer, 0.96 PFLOP/s; 503 before the scalar addresses, the loads spread over
+// the S^T block and the separate unmasked loop.  32x32x16 MFMAs (the same
+// time), three column tiles per wave (+13%) and 32-key tiles at three waves
+// per SIMD (+9%) were no better.
 constexpr int prefill_col_tiles_per_wave(int d, int w) { return w == 8 ? 1 : 2; }
 constexpr bool prefill_built(int d, int w) { return w == 4 || (w == 8 && d <= 128); }
 constexpr int prefill_key_tile(int d) { return d <= 128 ? kPrefillKeyTile : 32; }
 constexpr int prefill_unit_columns(int d) { return 16 * prefill_col_tiles_per_wave(d, 4) * 4; }
 static_assert(16 * 1 * 8 == 16 * 2 * 4, "both shapes cover the same unit columns");
+
 
 // LDS tile layout.  A K (or V) tile of KT rows is stored as CG column groups
 // (64 bytes = four 16-byte chunks of every row), group-major: byte
@@ -131,7 +145,9 @@ struct PrefillArgs {
   float scale_log2;
 };
 
-template <typename T, int D, int W>
+// B16: block sizes that are powers of two from 16 on (a tile's row blocks of
+// 16 keys then never cross a block).
+template <typename T, int D, int W, bool B16>
 __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W == 8 ? 4 : (D <= 128 ? 2 : 1)))) void paged_prefill_kernel(
     const int32_t* __restrict__ units,  // [n][LVAMD_PREFILL_FIELDS]
     const int32_t num_kv_heads, const PrefillArgs a) {
@@ -186,20 +202,33 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W == 8 ?
   // ---- tile loads.  Wave w loads row block w % RB of every tile, column
   // groups w / RB, w / RB + W / RB, ...; lane l the row 16 (w % RB) + l / 4
   // into chunk slot l % 4 of each group (chunk 4 cg + ((l % 4) ^ swz(row))):
-  // one table entry and one row address per tile.
-  const int lrow = 16 * (wave % RB) + (lane >> 2);
+  // one table entry and one row address per tensor and tile.
+  const int rb = wave % RB;
+  const int lrow = 16 * rb + (lane >> 2);
   const int lchunk = (lane & 3) ^ prefill_swz<W>(lrow);
-  // Fused append: keys at positions >= computed are this step's tokens, read
-  // from the input K/V; the unit that holds a token's own query (its first
-  // column) also writes the row to its pool slot, so no other launch appends.
+  // Keys at positions >= computed are this step's tokens, read from the input
+  // K/V (or from the pool when that already holds them).
   gptr<const T> const knew = a.k_new ? (gptr<const T>)(a.k_new) + (int64_t)kvh * a.kn_head_stride : nullptr;
   gptr<const T> const vnew = a.v_new ? (gptr<const T>)(a.v_new) + (int64_t)kvh * a.vn_head_stride : nullptr;
-  auto key_pos = [&](int t) -> int {
-    const int pos = (tile0 + t) * KT + lrow;
-    return pos < kmax ? pos : kmax - 1;  // rows past the piece read its last key (masked)
+  const int pool_end = knew != nullptr && computed < kmax ? computed : kmax;  // keys in the pool
+  auto logical_block = [&](int pos) -> int {
+    if constexpr (B16) return pos >> a.bs_shift;
+    return a.bs_shift >= 0 ? (pos >> a.bs_shift) : (pos / bs);
   };
-  auto logical_block = [&](int pos) -> int { return a.bs_shift >= 0 ? (pos >> a.bs_shift) : (pos / bs); };
-  auto load_entry = [&](int t) -> int { return table[logical_block(key_pos(t))]; };
+  // The key whose block's table entry this lane needs: its row's, or (B16) its
+  // row block's first.  Rows past the piece read its last key (masked).
+  auto key_pos = [&](int t) -> int {
+    const int pos = (tile0 + t) * KT + (B16 ? 16 * rb : lrow);
+    return pos < kmax ? pos : kmax - 1;
+  };
+  // The entry goes to a vector register (the empty asm keeps the compiler from
+  // making a uniform index's load scalar at once: it then waits for the load
+  // where it is issued, a round trip per tile).
+  auto load_entry = [&](int t) -> int {
+    int i = logical_block(key_pos(t));
+    asm("" : "+v"(i));
+    return table[i];
+  };
   // Tile 0's entry from the record (its rows lie in the tile's blocks, the
   // first of which is logical block key_begin / block_size).
   auto first_entry = [&]() -> int {
@@ -207,37 +236,93 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W == 8 ?
     const int k = logical_block(key_pos(0)) - logical_block(key_begin);
     return k == 0 ? first_blocks[0] : k == 1 ? first_blocks[1] : k == 2 ? first_blocks[2] : first_blocks[3];
   };
-  // Chunk of column group cg this lane copies (D = 80: the half-used last
-  // group's spare slots copy the row's last chunk again; nothing reads them).
+  // Chunk of column group cg this lane copies (a half-used last group's spare
+  // slots copy the row's last chunk again; nothing reads them).
   auto chunk_of = [&](int cg) -> int {
     const int ch = 4 * cg + lchunk;
     if constexpr (4 * CG > CPR) return ch < CPR ? ch : CPR - 1;
     return ch;
   };
-  // Issues tile t's loads into (kdst, vdst); te is the row's table entry.
-  auto issue_tile = [&](int t, int te, char* kdst, char* vdst) {
-    const int pos = key_pos(t);
-    const uint32_t slot = (uint32_t)te * (uint32_t)bs + (uint32_t)(pos - logical_block(pos) * bs);
-    const int64_t off = (int64_t)slot * row_elems + kvh * D;
+  // Byte addresses of this lane's K and V rows (of its chunk of column group 0
+  // when every group is whole) of tile t; te is the row's table entry.  A row
+  // block wholly in the pool or wholly in the step's input (nonnegative
+  // strides that fit 32 bits) takes a scalar base and a fixed lane offset; the
+  // block that holds the border, or the piece's end, an address per lane.
+  constexpr bool kWhole = 4 * CG == CPR;
+  const int lane_chunk = kWhole ? lchunk * 8 : 0;
+  const uint32_t pool_voff = (uint32_t)((lane >> 2) * (int)row_elems + lane_chunk) * 2u;
+  const bool fresh_rows = knew != nullptr && a.kn_tok_stride >= 0 && a.kn_tok_stride < (1 << 24) &&
+                          a.vn_tok_stride >= 0 && a.vn_tok_stride < (1 << 24);
+  const uint32_t kn_voff = (uint32_t)((lane >> 2) * (int)a.kn_tok_stride + lane_chunk) * 2u;
+  const uint32_t vn_voff = (uint32_t)((lane >> 2) * (int)a.vn_tok_stride + lane_chunk) * 2u;
+  struct Src {
+    gptr<const char> k, v;
+  };
+  auto address = [&](int t, int te) -> Src {
+    const int p0 = (tile0 + t) * KT + 16 * rb;
+    if constexpr (B16) {
+      if (p0 + 16 <= pool_end) {
+        const uint32_t s0 = (uint32_t)__builtin_amdgcn_readfirstlane(te) * (uint32_t)bs + (uint32_t)(p0 & (bs - 1));
+        const int64_t off = (int64_t)s0 * row_elems + kvh * D;
+        return {(gptr<const char>)(kbase + off) + pool_voff, (gptr<const char>)(vbase + off) + pool_voff};
+      }
+    }
+    if (fresh_rows && p0 >= computed && p0 + 16 <= kmax) {
+      const int64_t row = q_start + p0 - computed;
+      return {(gptr<const char>)(knew + row * a.kn_tok_stride) + kn_voff,
+              (gptr<const char>)(vnew + row * a.vn_tok_stride) + vn_voff};
+    }
+    const int raw = p0 + (lane >> 2);
+    const int pos = raw < kmax ? raw : kmax - 1;
+    const uint32_t sl = (uint32_t)te * (uint32_t)bs + (uint32_t)(pos - logical_block(pos) * bs);
+    const int64_t off = (int64_t)sl * row_elems + kvh * D;
     gptr<const T> kp = kbase + off;
     gptr<const T> vp = vbase + off;
-    bool append = false;
     if (knew != nullptr && pos >= computed) {
-      const int j = pos - computed;  // query index of the row's token
+      const int j = pos - computed;
       kp = knew + (int64_t)(q_start + j) * a.kn_tok_stride;
       vp = vnew + (int64_t)(q_start + j) * a.vn_tok_stride;
-      const int raw = (tile0 + t) * KT + lrow;
-      append = raw == pos && j * G >= col0;  // (j * G < col_end: pos < kmax <= kneed)
     }
-    const int lds_row = (wave % RB) * 1024;
-    for (int cg = wave / RB; cg < CG; cg += W / RB) {
-      const int ch = chunk_of(cg);
-      __builtin_amdgcn_global_load_lds((lds_gptr)(kp + ch * 8), (lds_lptr)(kdst + cg * GB + lds_row), 16, 0, 0);
-      __builtin_amdgcn_global_load_lds((lds_gptr)(vp + ch * 8), (lds_lptr)(vdst + cg * GB + lds_row), 16, 0, 0);
-      if (append) {
-        store16((gptr<T>)(kbase + off + ch * 8), load16(kp + ch * 8));
-        store16((gptr<T>)(vbase + off + ch * 8), load16(vp + ch * 8));
-      }
+    return {(gptr<const char>)(kp + lane_chunk), (gptr<const char>)(vp + lane_chunk)};
+  };
+  constexpr int CSTEP = W / RB;
+  constexpr int LPT = (CG + CSTEP - 1) / CSTEP;  // loads per lane, tensor and tile
+  // Load i of a tile's 2 LPT (K even, V odd) into (kdst, vdst).
+  auto issue_load = [&](const Src& x, int i, char* kdst, char* vdst) {
+    const int cg = wave / RB + (i >> 1) * CSTEP;
+    if (CG % CSTEP != 0 && cg >= CG) return;
+    const int off = kWhole ? cg * 64 : chunk_of(cg) * 16;
+    char* const dst = (i & 1 ? vdst : kdst) + rb * 1024 + cg * GB;
+    __builtin_amdgcn_global_load_lds((lds_gptr)((i & 1 ? x.v : x.k) + off), (lds_lptr)dst, 16, 0, 0);
+  };
+  auto issue_tile = [&](const Src& x, char* kdst, char* vdst) {
+#pragma unroll
+    for (int i = 0; i < 2 * LPT; ++i) issue_load(x, i, kdst, vdst);
+  };
+
+  // Fused append: writes tile t's rows of this step's tokens whose own query
+  // is in this unit (its first column) to their pool slots, each lane the
+  // chunks that it loaded into (ksrc, vsrc); no other workgroup writes the
+  // row.  (Copied from the input when the tile was issued, each chunk's load
+  // and store held the tile's own loads back: 32 shared-prefix trees, 8 layers,
+  // 220 against 204 us; four trees of 500-2,500 tokens 154 against 128.)  te:
+  // the rows' table entry.
+  auto append_rows = [&](int t, int te, const char* ksrc, const char* vsrc) {
+    const int p0 = (tile0 + t) * KT + 16 * rb;
+    if (knew == nullptr || p0 >= kmax || p0 + 15 < computed || (p0 + 15 - computed) * G < col0) return;
+    const int pos = p0 + (lane >> 2);
+    const int j = pos - computed;
+    if (pos >= kmax || j < 0 || j * G < col0) return;
+    const uint32_t sl = (uint32_t)te * (uint32_t)bs + (uint32_t)(pos - logical_block(pos) * bs);
+    const int64_t off = (int64_t)sl * row_elems + kvh * D;
+#pragma unroll
+    for (int i = 0; i < LPT; ++i) {
+      const int cg = wave / RB + i * CSTEP;
+      if (CG % CSTEP != 0 && cg >= CG) break;
+      const int at = rb * 1024 + cg * GB + lane * 16;
+      const int ch = chunk_of(cg) * 8;
+      store16((gptr<T>)(kbase + off + ch), *reinterpret_cast<const uint4*>(ksrc + at));
+      store16((gptr<T>)(vbase + off + ch), *reinterpret_cast<const uint4*>(vsrc + at));
     }
   };
 
@@ -304,38 +389,53 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W == 8 ?
   const int v_off1 = v_row * 64 + 16 * ((2 + (q4 >> 1)) ^ prefill_swz<W>(v_row)) + 8 * (q4 & 1);
 
   // ---- one tile of attention from LDS (t: tile of the piece)
-  auto compute_tile = [&](int tr, const char* kt, const char* vt) {
+  // MASKED: the tile may reach past the fully visible prefix.  (The unmasked
+  // copy, for the W = 4 shape's long loop, has no mask values merging into the
+  // scores' registers; it also issues the next tile's loads x, one per few
+  // MFMAs, so that the wave's matrix work does not wait behind eight loads.)
+  auto compute_tile = [&]<bool MASKED>(int tr, const char* kt, const char* vt, const Src x, char* kn, char* vn)
+      __attribute__((always_inline)) {
     const int t = tile0 + tr;
-    if (!wave_active || t * KT >= wave_kmax) return;
+    if (!wave_active || (MASKED && t * KT >= wave_kmax)) return;
     // S^T for each column tile, K chunks shared.  Each MFMA block runs at
     // raised wave priority: the SIMD's other wave then does its softmax
     // VALU work while this one feeds the matrix core, and the two phases
-    // overlap (measured 7% on a chunked-prefill step in both shapes).
-    // iglp_opt(0) asks the scheduler to interleave the block's LDS reads with
-    // its MFMAs (a further 4% in the 4-wave shape).
+    // overlap (measured 7% on a chunked-prefill step in both shapes).  LDS
+    // reads run LEAD operands ahead of the MFMAs: held there by scheduling
+    // barriers with two column tiles per wave (left alone, the scheduler
+    // hoists the reads and the registers spill), by iglp_opt(0) with one.
     __builtin_amdgcn_s_setprio(1);
-    __builtin_amdgcn_iglp_opt(0);
     f32x4 st[CT][KS];
-#pragma unroll
-    for (int ct = 0; ct < CT; ++ct)
-#pragma unroll
-      for (int s = 0; s < KS; ++s) st[ct][s] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int s = 0; s < KS; ++s)
-#pragma unroll
-      for (int kk = 0; kk < NCH; ++kk) {
+    if constexpr (W == 8) __builtin_amdgcn_iglp_opt(0);
+    {
+      constexpr int TOT = KS * NCH, LEAD = TOT < 3 ? TOT : 3;
+      static_assert(TOT >= 2 * LPT, "every load of the next tile has a place");
+      constexpr int LSTEP = TOT / (2 * LPT);
+      auto rd = [&](int i) -> uint4 {
+        const int s = i / NCH, kk = i % NCH;
         const int ch = kk * 4 + g;
-        const uint4 kc = ch < CPR ? *reinterpret_cast<const uint4*>(kt + kk * GB + s * 1024 + k_off) : zero_u4();
+        return ch < CPR ? *reinterpret_cast<const uint4*>(kt + kk * GB + s * 1024 + k_off) : zero_u4();
+      };
+      uint4 kf[LEAD];
 #pragma unroll
-        for (int ct = 0; ct < CT; ++ct) st[ct][s] = Mma<T>::qk(kc, qf[ct][kk], st[ct][s]);
+      for (int i = 0; i < LEAD; ++i) kf[i] = rd(i);
+      const f32x4 z = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int i = 0; i < TOT; ++i) {
+        const int s = i / NCH, kk = i % NCH;
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct) st[ct][s] = Mma<T>::qk(kf[i % LEAD], qf[ct][kk], kk == 0 ? z : st[ct][s]);
+        if (i + LEAD < TOT) kf[i % LEAD] = rd(i + LEAD);
+        if (W == 4 && !MASKED && i % LSTEP == 0 && i / LSTEP < 2 * LPT) issue_load(x, i / LSTEP, kn, vn);
+        if constexpr (W == 4) __builtin_amdgcn_sched_barrier(0);
       }
+    }
     __builtin_amdgcn_s_setprio(0);
-    const bool masked = t >= full_tiles;
     // Masks only past the fully visible prefix: one compare per score for a
     // linear request, the ancestor bits for a tree.  (A piece ends on a tile
     // boundary or at the unit's last key, so no unmasked tile reaches past
     // it; rows past kmax in a masked tile fail the visibility test.)
-    if (masked && !tree) {
+    if (MASKED && t >= full_tiles && !tree) {
       // Linear: key pos is visible to query qi iff pos <= computed + qi.
 #pragma unroll
       for (int ct = 0; ct < CT; ++ct) {
@@ -343,34 +443,39 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W == 8 ?
 #pragma unroll
         for (int s = 0; s < KS; ++s)
 #pragma unroll
-          for (int r = 0; r < 4; ++r)
-            if (16 * s + r > last) st[ct][s][r] = -INFINITY;
+          for (int r = 0; r < 4; ++r) st[ct][s][r] = 16 * s + r > last ? -INFINITY : st[ct][s][r];
       }
-    } else if (masked) {
+    } else if (MASKED && t >= full_tiles) {
       // Tree: keys before computed are visible, key j = pos - computed < q_len
-      // iff bit j of the query's ancestor row.  The tile's keys span at most
-      // NW words of the row; each column loads them once per tile, always in
-      // bounds (clamped), so the loads carry no condition.
-      constexpr int NW = KT / 32 + 1;
+      // iff bit j of the query's ancestor row.  Each column's bits of the
+      // tile's keys are funnel-shifted out of the row's words (loaded once
+      // per tile, in bounds), so a score takes two instructions: its bit,
+      // spread over the register, selects the score or -inf.  (Seven per
+      // score, and 455 per tile of two column tiles, with a word choice and
+      // two compares each.)
       const int j0 = t * KT - computed;  // j of the tile's first key
       const int w0 = j0 >> 5;            // (arithmetic: j0 may be negative)
 #pragma unroll
       for (int ct = 0; ct < CT; ++ct) {
-        uint32_t words[NW];
+        uint32_t bits[KT / 32];
+        uint32_t low = 0;
 #pragma unroll
-        for (int i = 0; i < NW; ++i) {
-          const int w = min(max(w0 + i, 0), vis_words - 1);
-          words[i] = tree_word ? vrow[ct] : a.vis[vis_off + qi[ct] * vis_words + w];
+        for (int i = 0; i <= KT / 32; ++i) {
+          const int wi = w0 + i;
+          const int left = q_len - 32 * wi;  // row bits from this word on
+          const uint32_t valid = left >= 32 ? ~0u : left <= 0 ? 0u : (1u << left) - 1;
+          const uint32_t row =
+              tree_word ? vrow[ct] : a.vis[vis_off + qi[ct] * vis_words + min(max(wi, 0), vis_words - 1)];
+          const uint32_t word = wi < 0 ? ~0u : row & valid;
+          if (i > 0) bits[i - 1] = __builtin_amdgcn_alignbit(word, low, j0 & 31) >> (4 * g);
+          low = word;
         }
 #pragma unroll
         for (int s = 0; s < KS; ++s)
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
-            const int j = j0 + 16 * s + 4 * g + r;
-            const int wi = (j >> 5) - w0;  // 0 .. NW - 1
-            const uint32_t word = wi == 0 ? words[0] : wi == 1 ? words[1] : words[NW - 1];
-            const bool vis = j < 0 || (j < q_len && ((word >> (j & 31)) & 1u));
-            if (!vis) st[ct][s][r] = -INFINITY;
+            const int seen = ((int)(bits[s >> 1] << (31 - 16 * (s & 1) - r))) >> 31;  // -1: visible
+            st[ct][s][r] = __uint_as_float((__float_as_uint(st[ct][s][r]) & seen) | (0xff800000u & ~seen));
           }
       }
     }
@@ -403,36 +508,41 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W == 8 ?
     }
     // O^T += V^T P^T: transpose reads shared by the column tiles.
     __builtin_amdgcn_s_setprio(1);
-    __builtin_amdgcn_iglp_opt(0);
-#pragma unroll
-    for (int h = 0; h < KS / 2; ++h)
-#pragma unroll
-      for (int ct = 0; ct < CT; ++ct) {
-        if constexpr (std::is_same<T, __bf16>::value) {
-          l_run[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, pb[ct][h], l_run[ct], 0, 0, 0);
-        } else {
-          l_run[ct] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ones, pb[ct][h], l_run[ct], 0, 0, 0);
-        }
-      }
-#pragma unroll
-    for (int h = 0; h < KS / 2; ++h)
-#pragma unroll
-      for (int n = 0; n < NT; ++n) {
+    if constexpr (W == 8) __builtin_amdgcn_iglp_opt(0);
+    {
+      constexpr int TOT = KS / 2 * NT, LEAD = TOT < 2 ? TOT : 2;
+      auto rd = [&](int i) -> V8 {
+        const int h = i / NT, n = i % NT;
         const int lo = (n & 1 ? v_off1 : v_off0) + (n >> 1) * GB + h * 32 * 64;
-        const int hi = lo + 16 * 64;
         const s16x4 v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t*)(vt + lo));
-        const s16x4 v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t*)(vt + hi));
+        const s16x4 v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t*)(vt + lo + 16 * 64));
         const s16x4 both[2] = {v0, v1};
-        const V8 av = bitcast<V8>(both);
-#pragma unroll
-        for (int ct = 0; ct < CT; ++ct) {
-          if constexpr (std::is_same<T, __bf16>::value) {
-            acc[ct][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, pb[ct][h], acc[ct][n], 0, 0, 0);
-          } else {
-            acc[ct][n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av, pb[ct][h], acc[ct][n], 0, 0, 0);
-          }
+        return bitcast<V8>(both);
+      };
+      auto mm = [&](V8 x, V8 y, f32x4 c) -> f32x4 {
+        if constexpr (std::is_same<T, __bf16>::value) {
+          return __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, y, c, 0, 0, 0);
+        } else {
+          return __builtin_amdgcn_mfma_f32_16x16x32_f16(x, y, c, 0, 0, 0);
         }
+      };
+      V8 vf[LEAD];
+#pragma unroll
+      for (int i = 0; i < LEAD; ++i) vf[i] = rd(i);
+#pragma unroll
+      for (int h = 0; h < KS / 2; ++h)
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct) l_run[ct] = mm(ones, pb[ct][h], l_run[ct]);
+      if constexpr (W == 4) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < TOT; ++i) {
+        const int h = i / NT, n = i % NT;
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct) acc[ct][n] = mm(vf[i % LEAD], pb[ct][h], acc[ct][n]);
+        if (i + LEAD < TOT) vf[i % LEAD] = rd(i + LEAD);
+        if constexpr (W == 4) __builtin_amdgcn_sched_barrier(0);
       }
+    }
     __builtin_amdgcn_s_setprio(0);
   };
 
@@ -445,22 +555,38 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W == 8 ?
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
     __builtin_amdgcn_s_barrier();
   };
-  int ea = first_entry(), eb = 0;
-  issue_tile(0, ea, klds0, vlds0);
-  if (ntiles > 1) ea = load_entry(1);
+  int here = first_entry(), next = 0;  // table entries of tiles t and t + 1
+  issue_tile(address(0, here), klds0, vlds0);
+  if (ntiles > 1) next = load_entry(1);
   tile_done();
-  // en: tile t+1's entry (in), ef: receives tile t+2's.
-  auto step = [&](int t, const char* kc, const char* vc, char* kn, char* vn, const int en, int& ef) {
-    // The entry load goes first: a wait for it then never waits for the
-    // tile's loads (the vector memory counter retires in issue order).
-    if (t + 2 < ntiles) ef = load_entry(t + 2);
-    if (t + 1 < ntiles) issue_tile(t + 1, en, kn, vn);
-    compute_tile(t, kc, vc);
+  auto step = [&]<bool MASKED>(int t, const char* kc, const char* vc, char* kn, char* vn)
+      __attribute__((always_inline)) {
+    const bool more = !MASKED || t + 1 < ntiles;
+    Src x = {nullptr, nullptr};
+    if (more) x = address(t + 1, next);
+    const int entry = here;
+    here = next;
+    // The entry load goes before the tile's loads: a wait for it then never
+    // waits for them (the vector memory counter retires in issue order).
+    if (!MASKED || t + 2 < ntiles) next = load_entry(t + 2);
+    if ((W == 8 || MASKED || !wave_active) && more) issue_tile(x, kn, vn);
+    // (After the tile's matrix work where the registers allow it.)
+    if constexpr (MASKED && W == 4) append_rows(t, entry, kc, vc);
+    compute_tile.template operator()<MASKED>(t, kc, vc, x, kn, vn);
+    if constexpr (MASKED && W == 8) append_rows(t, entry, kc, vc);
     tile_done();
   };
-  for (int t = 0; t < ntiles; t += 2) {
-    step(t, klds0, vlds0, klds1, vlds1, ea, eb);
-    if (t + 1 < ntiles) step(t + 1, klds1, vlds1, klds0, vlds0, eb, ea);
+  // Pairs of tiles that no column masks, that hold none of this unit's own
+  // tokens and that a tile follows; then the rest.
+  int t = 0;
+  const int nfull = min((tree ? computed : computed + col0 / G) / KT - tile0, ntiles - 1) - 1;
+  for (; t < nfull; t += 2) {
+    step.template operator()<false>(t, klds0, vlds0, klds1, vlds1);
+    step.template operator()<false>(t + 1, klds1, vlds1, klds0, vlds0);
+  }
+  for (; t < ntiles; t += 2) {
+    step.template operator()<true>(t, klds0, vlds0, klds1, vlds1);
+    if (t + 1 < ntiles) step.template operator()<true>(t + 1, klds1, vlds1, klds0, vlds0);
   }
 
   // ---- normalised output rows, or this piece's partials
@@ -491,18 +617,24 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W == 8 ?
   }
 }
 
+template <typename T, int D, int W>
+static int launch_prefill_w(dim3 grid, hipStream_t s, const int32_t* units, int32_t num_kv_heads, const PrefillArgs& a) {
+  if constexpr (prefill_built(D, W)) {
+    if (a.bs_shift >= 4) {
+      hipLaunchKernelGGL((paged_prefill_kernel<T, D, W, true>), grid, dim3(64 * W), 0, s, units, num_kv_heads, a);
+    } else {
+      hipLaunchKernelGGL((paged_prefill_kernel<T, D, W, false>), grid, dim3(64 * W), 0, s, units, num_kv_heads, a);
+    }
+    return launch_status();
+  }
+  return LVAMD_ERR_UNSUPPORTED;
+}
+
 template <typename T, int D>
 static int launch_prefill_d(int waves, dim3 grid, hipStream_t s, const int32_t* units, int32_t num_kv_heads,
                             const PrefillArgs& a) {
-  if (waves == 8) {
-    if constexpr (prefill_built(D, 8)) {
-      hipLaunchKernelGGL((paged_prefill_kernel<T, D, 8>), grid, dim3(512), 0, s, units, num_kv_heads, a);
-      return launch_status();
-    }
-    return LVAMD_ERR_UNSUPPORTED;
-  }
-  hipLaunchKernelGGL((paged_prefill_kernel<T, D, 4>), grid, dim3(256), 0, s, units, num_kv_heads, a);
-  return launch_status();
+  return waves == 8 ? launch_prefill_w<T, D, 8>(grid, s, units, num_kv_heads, a)
+                    : launch_prefill_w<T, D, 4>(grid, s, units, num_kv_heads, a);
 }
 
 template <typename T>
@@ -531,10 +663,10 @@ static int launch_prefill_t(int head_size, int waves, dim3 grid, hipStream_t s, 
 template <typename T, int D>
 static const void* prefill_fn(int waves) {
   if (waves == 8) {
-    if constexpr (prefill_built(D, 8)) return (const void*)&paged_prefill_kernel<T, D, 8>;
+    if constexpr (prefill_built(D, 8)) return (const void*)&paged_prefill_kernel<T, D, 8, true>;
     return nullptr;
   }
-  return (const void*)&paged_prefill_kernel<T, D, 4>;
+  return (const void*)&paged_prefill_kernel<T, D, 4, true>;
 }
 
 template <typename T>
@@ -592,7 +724,7 @@ extern "C" int lvamd_paged_prefill_resident_units(int32_t dtype, int32_t head_si
 
 extern "C" int lvamd_paged_prefill_waves_built(int32_t dtype, int32_t head_size, int32_t waves) {
   if (!prefill_supported(dtype, head_size)) return 0;
-  return (waves == 4 || (waves == 8 && head_size <= 128)) ? 1 : 0;
+  return (waves == 4 || (waves == 8 && head_size <= 128 )) ? 1 : 0;
 }
 
 extern "C" int lvamd_paged_prefill(const void* q, int64_t q_token_stride, int64_t q_head_stride,
