@@ -1505,9 +1505,21 @@ int64_t choose_col_tiles(const Requests& q, int64_t group, int64_t max_cols, int
   return four * cost4 < one ? 4 : 1;
 }
 
-// Prefill workgroup shape: 8 waves of one column tile when the units will
-// be split over the resident workgroups or are short (mean key tiles per
-// unit at most wide_max_tiles), else 4 waves of two column tiles.
+// Prefill workgroup shape: 8 waves of one column tile where a workgroup slot
+// has few key tiles (latency counts), else 4 waves of two column tiles (each
+// LDS read feeds two MFMAs).  With split-K the line is kWideShareTiles key
+// tiles per resident 8-wave workgroup; without (no resident count) it is a
+// mean of wide_max_tiles per unit.  Measured per step of 2-8 layers (28 / 4
+// heads, D 128 unless named), 8 waves / 4 waves, by tiles per slot: 0.8 (four
+// trees) 128 / 136 us, 3 (32 trees) 226 / 223, 4.5 (16 chunks of 64 over 500)
+// 248 / 250, 5.2 (1,000 over 1,000, D 64) 166 / 179, 7.3 (16 ragged prompts,
+// D 64) 122 / 145, 7.5 (16 of 300 over 300, 12 / 2 heads) 346 / 354, 7.2 (two
+// of 1,000) 359 / 349, 8.0 (eight of 512) 334 / 323, 11.5 (four of 200 over
+// 2K) 455 / 433, 15 (512 over 4K) 504 / 474, 57 (4,096) 596 / 545, 114 (two of
+// 512 over 16K) 1220 / 1116, 210 (2,048 over 14K) 1035 / 936; the other way
+// only 14.7 (eight of 128 over 2K) 520 / 539.
+constexpr int64_t kWideShareTiles = 8;
+
 int64_t choose_prefill_waves(const Requests& q, const PrefillParams& p, int64_t slots_per_head8, bool wide_built,
                              double wide_max_tiles) {
   if (!wide_built) return 4;
@@ -1515,8 +1527,8 @@ int64_t choose_prefill_waves(const Requests& q, const PrefillParams& p, int64_t 
   if (units.empty()) return 4;
   int64_t tile_sum = 0;
   for (const Unit& u : units) tile_sum += u.tiles;
-  const bool split = slots_per_head8 > 0 && (int64_t)units.size() < slots_per_head8;
-  return split || (double)tile_sum / (double)units.size() <= wide_max_tiles ? 8 : 4;
+  if (slots_per_head8 > 0) return tile_sum < kWideShareTiles * slots_per_head8 ? 8 : 4;
+  return (double)tile_sum / (double)units.size() <= wide_max_tiles ? 8 : 4;
 }
 
 template <typename T>
@@ -1732,7 +1744,7 @@ const char* plan_layer(const Requests& q, const int32_t* ids, int64_t nflat, con
     if (k[7] > 0) {
       waves = (k[7] == 8 && k[9]) ? 8 : 4;
     } else {
-      waves = choose_prefill_waves(q, p, k[5] ? k[14] / hkv : 0, k[9] != 0, wide_max);
+      waves = choose_prefill_waves(q, p, k[5] ? k[15] / hkv : 0, k[9] != 0, wide_max);
     }
     p.resident_per_head = (waves == 8 ? k[15] : k[14]) / hkv;
     p.slots_per_head = k[5] ? p.resident_per_head : 0;

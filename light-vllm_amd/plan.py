@@ -181,11 +181,12 @@ def choose_prefill_waves(
     *, q_lens: np.ndarray, computed: np.ndarray, rows: np.ndarray, group: int, columns: int, key_tokens: int,
     slots_per_head: int, wide_built: bool,
 ) -> int:
-    """Workgroup shape of the prefill kernel for these rows: 8 waves of one
-    column tile when the units will be split over the resident workgroups or
-    are short (mean key tiles per unit at most PREFILL_WIDE_MAX_TILES), where
-    latency hiding pays; else 4 waves of two column tiles, whose K/V LDS reads
-    each feed two MFMAs.  Measured per workload in the prefill kernel's notes.
+    """A first estimate of the prefill workgroup shape from the units' count
+    and mean length alone: 8 waves of one column tile when there are fewer
+    units than resident workgroups or they are short (mean key tiles per unit
+    at most PREFILL_WIDE_MAX_TILES), else 4 waves of two column tiles.  A
+    step's plan takes the native planner's rule, which weighs the key tiles
+    per resident workgroup where units may be split.
     """
 
     if not wide_built or not rows.any():
