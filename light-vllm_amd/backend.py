@@ -226,6 +226,7 @@ class HipPagedAttention:
         self._statics = backend.layer_statics(cache) if _raw_stream is not None else {}
         self._shape_bound: dict[tuple, tuple] = {}
         self._attend_tensors = backend._attend_tensors
+        self._attend_rotary = backend._attend_rotary
         self._attend_fn = backend._attend_fn
 
     @property
@@ -252,19 +253,24 @@ class HipPagedAttention:
             raise errors.KVCacheError(f"paged attention layer {layer_id!r} ran more than once")
         self._layer_ids.add(layer_id)
         # The common case in one native call (the host module's
-        # attend_tensors): it reads the tensors' dtype, device, shapes,
-        # strides and pointers, and launches when every rule holds (the
-        # layer's shapes, dtype and device, 16-byte rows); anything else, and
-        # rotary, takes the general path, which raises the first broken
-        # rule's message.
+        # attend_tensors, or attend_rotary): it reads the tensors' dtype,
+        # device, shapes, strides and pointers, and launches when every rule
+        # holds (the layer's shapes, dtype and device, 16-byte rows); anything
+        # else takes the general path, which raises the first broken rule's
+        # message.  (Rotary steps on the general path cost 25 us of host time
+        # per layer, more than their kernels.)
         static = self._statics.get(layer_id)
-        if static is not None and rotary is None:
+        if static is not None and (rotary is None or (type(rotary) is tuple and len(rotary) == 2)):
             bound = self._shape_bound.get(static.shape)
             if bound is None:
                 bound = self._bind_shape(static)
             index = static.index
-            status = self._attend_tensors(bound[0], static.k_pool, static.v_pool, bound[1] + index * bound[2],
-                                          query, key, value, scale)
+            if rotary is None:
+                status = self._attend_tensors(bound[0], static.k_pool, static.v_pool, bound[1] + index * bound[2],
+                                              query, key, value, scale)
+            else:
+                status = self._attend_rotary(bound[0], static.k_pool, static.v_pool, bound[1] + index * bound[2],
+                                             query, key, value, scale, rotary[0], rotary[1], bound[5], bound[6])
             if status == 0:
                 return bound[3][index]
             if status != _NOT_FAST:
@@ -274,7 +280,8 @@ class HipPagedAttention:
     def _bind_shape(self, static) -> tuple:
         """The fast path's facts for the layers of one shape in this step:
         (the shape's facts for attend_tensors, the output slab's address,
-        its bytes per layer, the per-layer output views).
+        its bytes per layer, the per-layer output views, the launch, the
+        rotary append's facts, the rotated-query buffer of a stream).
 
         Outputs are views of one tensor per layer shape and step, made at the
         first layer of that shape (one allocation for the step's layers in
@@ -299,8 +306,20 @@ class HipPagedAttention:
             static.device_index, static.element_size, tokens, spec.num_query_heads, spec.num_kv_heads,
             spec.head_size, _raw_stream,
         )
+        rotated: dict[int, Tensor] = {}
+
+        def rotated_queries(stream: int) -> int:
+            # One buffer per stream of the step: a stream's layers run in
+            # order, so each layer's attention has read it before the next
+            # layer's rotary append writes it.
+            buffer = rotated.get(stream)
+            if buffer is None:
+                buffer = rotated[stream] = torch.empty((tokens, spec.num_query_heads, spec.head_size),
+                                                       dtype=static.dtype, device=static.device)
+            return buffer.data_ptr()
+
         bound = (facts, slab.data_ptr(), tokens * spec.num_query_heads * spec.head_size * static.element_size,
-                 views, launch)
+                 views, launch, (self._backend._rotary_fn, self._plan.slots_ptr, launch.dtype), rotated_queries)
         self._shape_bound[static.shape] = bound
         return bound
 
@@ -512,6 +531,8 @@ class HipPagedAttentionBackend:
         # What every context's fast forward calls, looked up once.
         self._lib = native.load()
         self._attend_tensors = native.host().attend_tensors
+        self._attend_rotary = native.host().attend_rotary
+        self._rotary_fn = native.rotary_entry()
         self._attend_fn = native.attention_entry()
 
     def prefill_columns(self, code: int, head_size: int) -> int:

@@ -2189,49 +2189,165 @@ int tensor_facts(PyObject* t, PyObject* dtype, long device, int64_t n0, int64_t 
   return 1;
 }
 
-PyObject* attend_tensors(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
-  if (!want_args(nargs, 8, "attend_tensors")) return nullptr;
+// The layer's tensors and launch facts of attend_tensors and attend_rotary.
+struct AttendCall {
+  int64_t f[12];  // the shape facts' integers
+  int64_t k_pool, v_pool, out, stream;
+  int64_t qp, qs0, qs1, kp, ks0, ks1, vp, vs0, vs1;
+  double scale;
+};
+
+// args: shape, key_pool, value_pool, out, q, k, v, scale.  1: every rule of the
+// fast path holds (call filled), 0: one does not, -1: a Python error.
+int attend_call(PyObject* const* args, const char* name, AttendCall* c) {
   PyObject* b = args[0];
   if (!PyTuple_Check(b) || PyTuple_GET_SIZE(b) != 12) {
-    PyErr_SetString(PyExc_ValueError, "attend_tensors: shape facts must be a 12-tuple");
-    return nullptr;
+    PyErr_Format(PyExc_ValueError, "%s: shape facts must be a 12-tuple", name);
+    return -1;
   }
-  int64_t f[12];
   for (int i = 0; i < 12; ++i) {
     if (i == 4 || i == 11) continue;
-    f[i] = (int64_t)PyLong_AsLongLong(PyTuple_GET_ITEM(b, i));
+    c->f[i] = (int64_t)PyLong_AsLongLong(PyTuple_GET_ITEM(b, i));
   }
-  const int64_t k_pool = (int64_t)PyLong_AsLongLong(args[1]);
-  const int64_t v_pool = (int64_t)PyLong_AsLongLong(args[2]);
-  const int64_t out = (int64_t)PyLong_AsLongLong(args[3]);
-  if (PyErr_Occurred()) return nullptr;
+  c->k_pool = (int64_t)PyLong_AsLongLong(args[1]);
+  c->v_pool = (int64_t)PyLong_AsLongLong(args[2]);
+  c->out = (int64_t)PyLong_AsLongLong(args[3]);
+  if (PyErr_Occurred()) return -1;
   PyObject* dtype = PyTuple_GET_ITEM(b, 4);
-  const long device = (long)f[5];
-  const int64_t es = f[6], tokens = f[7], hq = f[8], hkv = f[9], d = f[10];
-  int64_t qp, qs0, qs1, kp, ks0, ks1, vp, vs0, vs1;
-  int r = tensor_facts(args[4], dtype, device, tokens, hq, d, es, &qp, &qs0, &qs1);
-  if (r == 1) r = tensor_facts(args[5], dtype, device, tokens, hkv, d, es, &kp, &ks0, &ks1);
-  if (r == 1) r = tensor_facts(args[6], dtype, device, tokens, hkv, d, es, &vp, &vs0, &vs1);
-  if (r < 0) return nullptr;
-  if (r == 0) return PyLong_FromLong(kNotFast);
-  const double scale = PyFloat_AsDouble(args[7]);
-  if (PyErr_Occurred()) return nullptr;
+  const long device = (long)c->f[5];
+  const int64_t es = c->f[6], tokens = c->f[7], hq = c->f[8], hkv = c->f[9], d = c->f[10];
+  int r = tensor_facts(args[4], dtype, device, tokens, hq, d, es, &c->qp, &c->qs0, &c->qs1);
+  if (r == 1) r = tensor_facts(args[5], dtype, device, tokens, hkv, d, es, &c->kp, &c->ks0, &c->ks1);
+  if (r == 1) r = tensor_facts(args[6], dtype, device, tokens, hkv, d, es, &c->vp, &c->vs0, &c->vs1);
+  if (r != 1) return r;
+  c->scale = PyFloat_AsDouble(args[7]);
+  if (PyErr_Occurred()) return -1;
   PyObject* dev = PyLong_FromLong(device);
-  if (dev == nullptr) return nullptr;
+  if (dev == nullptr) return -1;
   PyObject* stream = PyObject_CallOneArg(PyTuple_GET_ITEM(b, 11), dev);
   Py_DECREF(dev);
-  if (stream == nullptr) return nullptr;
-  const int64_t sp = PyLong_AsLongLong(stream);
+  if (stream == nullptr) return -1;
+  c->stream = PyLong_AsLongLong(stream);
   Py_DECREF(stream);
-  if (PyErr_Occurred()) return nullptr;
-  if (f[0] == 0 || f[1] == 0) {
-    PyErr_SetString(PyExc_ValueError, "attend_tensors: null function or plan");
+  if (PyErr_Occurred()) return -1;
+  if (c->f[0] == 0 || c->f[1] == 0) {
+    PyErr_Format(PyExc_ValueError, "%s: null function or plan", name);
+    return -1;
+  }
+  return 1;
+}
+
+void* as_ptr(int64_t v) { return reinterpret_cast<void*>((intptr_t)v); }
+
+PyObject* attend_tensors(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  if (!want_args(nargs, 8, "attend_tensors")) return nullptr;
+  AttendCall c;
+  const int r = attend_call(args, "attend_tensors", &c);
+  if (r < 0) return nullptr;
+  if (r == 0) return PyLong_FromLong(kNotFast);
+  const AttendFn fn = reinterpret_cast<AttendFn>((intptr_t)c.f[0]);
+  const int status = fn(as_ptr(c.f[1]), as_ptr(c.qp), c.qs0, c.qs1, as_ptr(c.kp), c.ks0, c.ks1, as_ptr(c.vp), c.vs0,
+                        c.vs1, as_ptr(c.k_pool), as_ptr(c.v_pool), as_ptr(c.out), c.f[2], c.f[3], (float)c.scale,
+                        as_ptr(c.stream));
+  return PyLong_FromLong(status);
+}
+
+// ---------------------------------------------------------------------------
+// attend_rotary(shape, key_pool, value_pool, out, q, k, v, scale, cosines,
+//               sines, (rotary fn, slots, dtype code), rotated(stream)) -> status,
+// or kNotFast
+//
+// attend_tensors for forward(..., rotary=): lvamd_kv_append_rotary (fn: its
+// address) into the layer's pools and the rotated-query buffer, then
+// lvamd_paged_attention on those queries with nothing left to append.
+// rotated(stream) gives the address of a [tokens][query heads][head size]
+// buffer for launches on that stream.  Cosines and sines are [tokens, head
+// size] rows of the layer's dtype and device with contiguous elements;
+// anything else, or a status of the rotary launch, returns kNotFast.
+// ---------------------------------------------------------------------------
+typedef int (*RotaryFn)(const void*, int64_t, int64_t, void*, int64_t, int64_t, const void*, int64_t, int64_t,
+                        const void*, int64_t, int64_t, const void*, int64_t, const void*, int64_t, void*, void*,
+                        const void*, int64_t, int32_t, int32_t, int32_t, int32_t, void*);
+
+// 1: t is a [n0, n1] tensor of the dtype and device with contiguous rows, 0:
+// it is not, -1: a Python error.
+int row_facts(PyObject* t, PyObject* dtype, long device, int64_t n0, int64_t n1, int64_t* ptr, int64_t* s0) {
+  PyObject* dt = PyObject_GetAttr(t, g_str_dtype);
+  if (dt == nullptr) return -1;
+  Py_DECREF(dt);
+  if (dt != dtype) return 0;
+  PyObject* dev = PyObject_CallMethodNoArgs(t, g_str_get_device);
+  if (dev == nullptr) return -1;
+  const long at = PyLong_AsLong(dev);
+  Py_DECREF(dev);
+  PyObject* shape = PyObject_GetAttr(t, g_str_shape);
+  if (shape == nullptr) return -1;
+  const bool fits = PyTuple_Check(shape) && PyTuple_GET_SIZE(shape) == 2 &&
+                    PyLong_AsLongLong(PyTuple_GET_ITEM(shape, 0)) == n0 &&
+                    PyLong_AsLongLong(PyTuple_GET_ITEM(shape, 1)) == n1;
+  Py_DECREF(shape);
+  if (PyErr_Occurred()) return -1;
+  if (!fits || at != device) return 0;
+  PyObject* stride = PyObject_CallMethodNoArgs(t, g_str_stride);
+  if (stride == nullptr) return -1;
+  int64_t st[2] = {0, 0};
+  if (PyTuple_Check(stride) && PyTuple_GET_SIZE(stride) == 2)
+    for (int i = 0; i < 2; ++i) st[i] = PyLong_AsLongLong(PyTuple_GET_ITEM(stride, i));
+  Py_DECREF(stride);
+  if (PyErr_Occurred()) return -1;
+  if (st[1] != 1) return 0;
+  PyObject* dp = PyObject_CallMethodNoArgs(t, g_str_data_ptr);
+  if (dp == nullptr) return -1;
+  *ptr = PyLong_AsLongLong(dp);
+  Py_DECREF(dp);
+  if (PyErr_Occurred()) return -1;
+  *s0 = st[0];
+  return 1;
+}
+
+PyObject* attend_rotary(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  if (!want_args(nargs, 12, "attend_rotary")) return nullptr;
+  AttendCall c;
+  int64_t cp, cs0, sp, ss0;
+  int r = attend_call(args, "attend_rotary", &c);
+  if (r == 1) r = row_facts(args[8], PyTuple_GET_ITEM(args[0], 4), (long)c.f[5], c.f[7], c.f[10], &cp, &cs0);
+  if (r == 1) r = row_facts(args[9], PyTuple_GET_ITEM(args[0], 4), (long)c.f[5], c.f[7], c.f[10], &sp, &ss0);
+  if (r < 0 && (PyErr_ExceptionMatches(PyExc_AttributeError) || PyErr_ExceptionMatches(PyExc_TypeError))) {
+    PyErr_Clear();  // an argument that is no tensor: the general path's message
+    r = 0;
+  }
+  if (r < 0) return nullptr;
+  if (r == 0) return PyLong_FromLong(kNotFast);
+  const int64_t tokens = c.f[7], hq = c.f[8], hkv = c.f[9], d = c.f[10];
+  PyObject* t = args[10];
+  if (!PyTuple_Check(t) || PyTuple_GET_SIZE(t) != 3) {
+    PyErr_SetString(PyExc_ValueError, "attend_rotary: rotary facts must be a 3-tuple");
     return nullptr;
   }
-  auto ptr = [](int64_t v) { return reinterpret_cast<void*>((intptr_t)v); };
-  const AttendFn fn = reinterpret_cast<AttendFn>((intptr_t)f[0]);
-  const int status = fn(ptr(f[1]), ptr(qp), qs0, qs1, ptr(kp), ks0, ks1, ptr(vp), vs0, vs1, ptr(k_pool), ptr(v_pool),
-                        ptr(out), f[2], f[3], (float)scale, ptr(sp));
+  int64_t f[3];
+  for (int i = 0; i < 3; ++i) f[i] = PyLong_AsLongLong(PyTuple_GET_ITEM(t, i));
+  if (PyErr_Occurred()) return nullptr;
+  if (f[0] == 0) {
+    PyErr_SetString(PyExc_ValueError, "attend_rotary: null function");
+    return nullptr;
+  }
+  PyObject* key = PyLong_FromLongLong(c.stream);
+  if (key == nullptr) return nullptr;
+  PyObject* buffer = PyObject_CallOneArg(args[11], key);
+  Py_DECREF(key);
+  if (buffer == nullptr) return nullptr;
+  void* const rotated = as_ptr(PyLong_AsLongLong(buffer));
+  Py_DECREF(buffer);
+  if (PyErr_Occurred()) return nullptr;
+  const RotaryFn rotate = reinterpret_cast<RotaryFn>((intptr_t)f[0]);
+  const int64_t rs0 = hq * d, rs1 = d;
+  if (rotate(as_ptr(c.qp), c.qs0, c.qs1, rotated, rs0, rs1, as_ptr(c.kp), c.ks0, c.ks1, as_ptr(c.vp), c.vs0, c.vs1,
+             as_ptr(cp), cs0, as_ptr(sp), ss0, as_ptr(c.k_pool), as_ptr(c.v_pool), as_ptr(f[1]), tokens, (int32_t)hq,
+             (int32_t)hkv, (int32_t)d, (int32_t)f[2], as_ptr(c.stream)) != 0)
+    return PyLong_FromLong(kNotFast);
+  const AttendFn fn = reinterpret_cast<AttendFn>((intptr_t)c.f[0]);
+  const int status = fn(as_ptr(c.f[1]), rotated, rs0, rs1, nullptr, 0, 0, nullptr, 0, 0, as_ptr(c.k_pool),
+                        as_ptr(c.v_pool), as_ptr(c.out), c.f[2], c.f[3], (float)c.scale, as_ptr(c.stream));
   return PyLong_FromLong(status);
 }
 
@@ -2250,6 +2366,8 @@ PyMethodDef kMethods[] = {
     {"attend", (PyCFunction)(void (*)(void))attend, METH_FASTCALL, "one layer's lvamd_paged_attention call"},
     {"attend_tensors", (PyCFunction)(void (*)(void))attend_tensors, METH_FASTCALL,
      "forward's fast path: tensor rules and the lvamd_paged_attention call"},
+    {"attend_rotary", (PyCFunction)(void (*)(void))attend_rotary, METH_FASTCALL,
+     "forward's fast path with rotary: the rotary append, then lvamd_paged_attention"},
     {nullptr, nullptr, 0, nullptr},
 };
 

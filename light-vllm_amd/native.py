@@ -282,6 +282,12 @@ def attention_entry() -> int:
     return ctypes.cast(load().lvamd_paged_attention, ctypes.c_void_p).value
 
 
+def rotary_entry() -> int:
+    """Address of ``lvamd_kv_append_rotary``, for the host module's ``attend_rotary``."""
+
+    return ctypes.cast(load().lvamd_kv_append_rotary, ctypes.c_void_p).value
+
+
 def check(status: int, what: str) -> None:
     if status != 0:
         message = load().lvamd_status_string(status).decode()
