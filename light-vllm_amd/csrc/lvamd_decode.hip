@@ -84,7 +84,7 @@ struct DecodeArgs {
   int32_t num_kv_heads;
   int32_t group;
   int32_t block_size;
-  int32_t bs_shift;  // log2(block_size) when a power of two, else -1
+  FastDiv by_block, by_group;  // / block_size, / group
   float scale_log2;
 };
 
@@ -249,7 +249,7 @@ __device__ __forceinline__ void merge_workgroup(const DecodeArgs& a, const float
       for (int e = 0; e < 4; ++e) o[e] += wt * (held ? row[i][e] : 0.f);
     }
     const float inv = lsum > 0.f ? 1.f / lsum : 0.f;
-    const int qi = col / a.group;
+    const int qi = fast_div(col, a.by_group);
     const int qhead = kvh * a.group + (col - qi * a.group);
     T* orow = static_cast<T*>(a.out) + (int64_t)(q_start + qi) * a.out_tok_stride + (int64_t)qhead * a.out_head_stride;
 #pragma unroll
@@ -264,7 +264,9 @@ template <typename T, int D, int CTW, int WG>
 __global__ __launch_bounds__(64 * WG) void paged_decode_kernel(
     const int32_t* __restrict__ wave_first,  // [waves_per_head + 1]
     const int32_t* __restrict__ pieces,      // [n_pieces][LVAMD_PIECE_FIELDS]
-    const int32_t waves_per_head, const DecodeArgs a) {
+    const int32_t waves_per_head,
+    const uint32_t wg_magic, const int32_t wg_shift,  // / workgroups per head
+    const DecodeArgs a) {
   using S = TileShape<T, D>;
   using DT = DecodeTile<T, D, CTW>;
   constexpr int E16 = S::E16, NCH = S::NCH, NT = S::NT, CPR = S::CPR;
@@ -309,7 +311,7 @@ __global__ __launch_bounds__(64 * WG) void paged_decode_kernel(
   // of WG waves).
   constexpr int kWG = WG;
   const int wg_per_head = waves_per_head / kWG;
-  const int kvh = blockIdx.x / wg_per_head;
+  const int kvh = fast_div((int)blockIdx.x, wg_magic, wg_shift);
   const int w = (blockIdx.x - kvh * wg_per_head) * kWG + wid;
   // The workgroup split holds one record per wave (wave w's at index w; an
   // idle wave's has request -1), so no wave_first lookup delays it.
@@ -376,9 +378,7 @@ __global__ __launch_bounds__(64 * WG) void paged_decode_kernel(
   gptr<const T> const vnew =
       a.v_new ? (gptr<const T>)(a.v_new) + (int64_t)kvh * a.vn_head_stride : nullptr;
 
-  auto logical_block = [&](int pos) -> int {
-    return a.bs_shift >= 0 ? (pos >> a.bs_shift) : (pos / a.block_size);
-  };
+  auto logical_block = [&](int pos) -> int { return fast_div(pos, a.by_block); };
 
   // Block-table slice of a piece: loaded into registers (lane i holds entries
   // i + 64j), stored to LDS when the piece's first tile is issued.
@@ -402,7 +402,7 @@ __global__ __launch_bounds__(64 * WG) void paged_decode_kernel(
     const int col = (x.cgroup * CTW + ct) * 16 + l16;
     c.ok = col < ncols;
     const int colc = c.ok ? col : ncols - 1;
-    c.qi = colc / G;
+    c.qi = fast_div(colc, a.by_group);
     c.qhead = kvh * G + (colc - c.qi * G);
     c.lin_last = x.computed + c.qi;
     c.vrow = (x.vis_off >= 0) ? a.vis + x.vis_off + (int64_t)c.qi * x.vis_words : nullptr;
@@ -427,11 +427,13 @@ __global__ __launch_bounds__(64 * WG) void paged_decode_kernel(
   // Issue one TT-token tile of piece x (table slice in tab[tb]): K chunks and
   // V chunks into registers.  Positions past the piece read its last row
   // (finite data, masked to probability 0, already in cache).  All row
-  // offsets are read from LDS before any load is issued.  fresh[s] is the
-  // pool offset of row group s's row when this tile must append it, else -1.
+  // offsets are read from LDS before any load is issued.  Returns whether the
+  // tile reaches this step's tokens; if so, fresh[s] is the pool offset of row
+  // group s's row when this tile must append it, else -1.
   auto issue_tile_ids = [&](const Piece& x, int t0, auto block_id, uint4 (&kdst)[SUB][NCH],
-                            uint4 (&vdst)[SUB][NCH], int64_t (&fresh)[FR]) {
+                            uint4 (&vdst)[SUB][NCH], int64_t (&fresh)[FR]) -> bool {
     const int lb0 = logical_block(x.tok_begin);
+    const bool reaches = knew != nullptr && min(t0 + TT, x.tok_end) > x.computed;
     if constexpr (LINES) {
       // Line order: entry i is chunk lane % CPR of row RPI * i + lane / CPR.
       constexpr int RPI = DT::RPI;
@@ -446,12 +448,18 @@ __global__ __launch_bounds__(64 * WG) void paged_decode_kernel(
         const int64_t off = ((int64_t)block_id(lb - lb0) * a.block_size + (pc - lb * a.block_size)) * row_elems;
         kp[i] = kbase + off;
         vp[i] = vbase + off;
-        fresh[i] = -1;
-        if (knew != nullptr && pc >= x.computed) {
+        fresh[i] = off;
+      }
+      if (reaches) {
+#pragma unroll
+        for (int i = 0; i < FR; ++i) {
+          const int pos = t0 + RPI * i + lane / CPR;
+          const int pc = pos < x.tok_end ? pos : x.tok_end - 1;
+          const bool isnew = pc >= x.computed;
           const int64_t t = x.q_start + (pc - x.computed);
-          kp[i] = knew + t * a.kn_tok_stride;
-          vp[i] = vnew + t * a.vn_tok_stride;
-          if (x.cgroup == 0 && pc == pos) fresh[i] = off;
+          kp[i] = isnew ? knew + t * a.kn_tok_stride : kp[i];
+          vp[i] = isnew ? vnew + t * a.vn_tok_stride : vp[i];
+          if (!isnew || x.cgroup != 0 || pc != pos) fresh[i] = -1;
         }
       }
 #pragma unroll
@@ -459,7 +467,7 @@ __global__ __launch_bounds__(64 * WG) void paged_decode_kernel(
         kdst[i / NCH][i % NCH] = load16_stream(kp[i] + c * E16);
         vdst[i / NCH][i % NCH] = load16_stream(vp[i] + c * E16);
       }
-      return;
+      return reaches;
     }
     gptr<const T> kp[SUB];
     gptr<const T> vp[SUB];
@@ -471,12 +479,18 @@ __global__ __launch_bounds__(64 * WG) void paged_decode_kernel(
       const int64_t off = ((int64_t)block_id(lb - lb0) * a.block_size + (pc - lb * a.block_size)) * row_elems;
       kp[s] = kbase + off;
       vp[s] = vbase + off;
-      fresh[s] = -1;
-      if (knew != nullptr && pc >= x.computed) {
+      fresh[s] = off;
+    }
+    if (reaches) {
+#pragma unroll
+      for (int s = 0; s < SUB; ++s) {
+        const int pos = t0 + 16 * s + l16;
+        const int pc = pos < x.tok_end ? pos : x.tok_end - 1;
+        const bool isnew = pc >= x.computed;
         const int64_t t = x.q_start + (pc - x.computed);
-        kp[s] = knew + t * a.kn_tok_stride;
-        vp[s] = vnew + t * a.vn_tok_stride;
-        if (x.cgroup == 0 && pc == pos) fresh[s] = off;
+        kp[s] = isnew ? knew + t * a.kn_tok_stride : kp[s];
+        vp[s] = isnew ? vnew + t * a.vn_tok_stride : vp[s];
+        if (!isnew || x.cgroup != 0 || pc != pos) fresh[s] = -1;
       }
     }
 #pragma unroll
@@ -492,10 +506,11 @@ __global__ __launch_bounds__(64 * WG) void paged_decode_kernel(
           vdst[s][kk] = zero_u4();
         }
       }
+    return reaches;
   };
   auto issue_tile = [&](const Piece& x, int tb, int t0, uint4 (&kdst)[SUB][NCH], uint4 (&vdst)[SUB][NCH],
-                        int64_t (&fresh)[FR]) {
-    issue_tile_ids(x, t0, [&](int rel) { return tab[tb][rel]; }, kdst, vdst, fresh);
+                        int64_t (&fresh)[FR]) -> bool {
+    return issue_tile_ids(x, t0, [&](int rel) { return tab[tb][rel]; }, kdst, vdst, fresh);
   };
   // Append the tile's fresh rows to the pool (bit-exact row copies).
   auto store_fresh = [&](const uint4 (&kr)[SUB][NCH], const uint4 (&vr)[SUB][NCH], const int64_t (&fresh)[FR]) {
@@ -568,6 +583,7 @@ __global__ __launch_bounds__(64 * WG) void paged_decode_kernel(
   int tc[TAB_PER_LANE];
   const int first_span = logical_block(min(cur.tok_begin + TT, cur.tok_end) - 1) - logical_block(cur.tok_begin);
   const bool direct = first_span < kPieceBlocks;
+  bool reaches0;
   if (direct) {
     if constexpr (WG == 1) {
       const int32_t* ids = pieces + (int64_t)p * LVAMD_PIECE_FIELDS + kPieceBlockField;
@@ -575,7 +591,7 @@ __global__ __launch_bounds__(64 * WG) void paged_decode_kernel(
       for (int i = 0; i < kPieceBlocks; ++i) first_ids[i] = ids[i];
     }
     const int b0 = first_ids[0], b1 = first_ids[1], b2 = first_ids[2], b3 = first_ids[3], b4 = first_ids[4];
-    issue_tile_ids(
+    reaches0 = issue_tile_ids(
         cur, cur.tok_begin,
         [&](int rel) { return rel == 0 ? b0 : rel == 1 ? b1 : rel == 2 ? b2 : rel == 3 ? b3 : b4; }, ka, vr0,
         fresh0);
@@ -583,7 +599,7 @@ __global__ __launch_bounds__(64 * WG) void paged_decode_kernel(
   } else {
     load_table(cur, tc);
     store_table(tb, tc);
-    issue_tile(cur, tb, cur.tok_begin, ka, vr0, fresh0);
+    reaches0 = issue_tile(cur, tb, cur.tok_begin, ka, vr0, fresh0);
   }
   load_q(cur, qf);
   bool have_nxt = WG == 1 && p + 1 < p_end;
@@ -596,7 +612,7 @@ __global__ __launch_bounds__(64 * WG) void paged_decode_kernel(
   }
   if (direct) store_table(tb, tc);
   stage_v(vlds_a, vr0, ka);
-  store_fresh(ka, vr0, fresh0);
+  if (reaches0) store_fresh(ka, vr0, fresh0);
 
   LaneCol lc[CTW];
   float m_run[CTW];  // per-column base (log2 domain), uniform across the column's lanes
@@ -652,14 +668,15 @@ __global__ __launch_bounds__(64 * WG) void paged_decode_kernel(
     uint4 vr[SUB][NCH];
     int64_t fresh[FR];
     const bool issued = next_in_cur || have_nxt;
+    bool reaches = false;
     if (next_in_cur) {
-      issue_tile(cur, tb, nt0, kx, vr, fresh);
+      reaches = issue_tile(cur, tb, nt0, kx, vr, fresh);
     } else if (have_nxt) {
       if (!nxt_stored) {
         store_table(tb ^ 1, tn);
         nxt_stored = true;
       }
-      issue_tile(nxt, tb ^ 1, nxt.tok_begin, kx, vr, fresh);
+      reaches = issue_tile(nxt, tb ^ 1, nxt.tok_begin, kx, vr, fresh);
     }
 
     // S^T tiles: rows = TT tokens (16-row groups), columns = this lane's
@@ -811,7 +828,7 @@ __global__ __launch_bounds__(64 * WG) void paged_decode_kernel(
     // and its fresh rows into the pool.
     if (issued) {
       stage_v(vx, vr, kx);
-      store_fresh(kx, vr, fresh);
+      if (reaches) store_fresh(kx, vr, fresh);
     }
     if (next_in_cur) t0 = nt0;
     return !next_in_cur;
@@ -970,6 +987,7 @@ struct MergeArgs {
   const float* part_ml;
   void* out;
   int64_t out_tok_stride, out_head_stride;
+  FastDiv by_group;  // / group
 };
 
 constexpr int kMergeRoundTrip = 16;  // partials a wave requests at once
@@ -991,6 +1009,7 @@ __global__ __launch_bounds__(64 * merge_waves(P)) void paged_merge_kernel(
     const int32_t groups,              // workgroups (of merge_columns columns) per (job, kv head)
     const int32_t num_kv_heads, const int32_t group,
     const int32_t col_tiles,           // column tiles per partial slot (the decode launch's)
+    const uint32_t groups_magic, const int32_t groups_shift, const uint32_t heads_magic, const int32_t heads_shift,
     const MergeArgs a) {
   using S = MergeShape<T, D>;
   constexpr int EPC = S::EPC, MCP = kMergeRoundTrip;
@@ -999,9 +1018,9 @@ __global__ __launch_bounds__(64 * merge_waves(P)) void paged_merge_kernel(
   const int cols = 16 * col_tiles;  // columns per partial slot
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int lane = threadIdx.x & 63;
-  const int jh = (int)blockIdx.x / groups;
+  const int jh = fast_div((int)blockIdx.x, groups_magic, groups_shift);
   const int c0 = ((int)blockIdx.x - jh * groups) * merge_columns<T, D, P> + (P == 1 ? wave * S::CW : 0);
-  const int job = jh / Hkv;
+  const int job = fast_div(jh, heads_magic, heads_shift);
   const int kvh = jh - job * Hkv;
   const int32_t* jb = jobs + (int64_t)job * LVAMD_MERGE_FIELDS;
   const int cgroup = jb[1], slot0 = jb[2], np = jb[3], q_start = jb[4], q_len = jb[5];
@@ -1011,7 +1030,7 @@ __global__ __launch_bounds__(64 * merge_waves(P)) void paged_merge_kernel(
   const int c = c0 + lane / S::LPC;
   const bool act = c < col_end && ch < S::CPR;
   const int col = cgroup * cols + (c < col_end ? c : c0);
-  const int qi = col / G;
+  const int qi = fast_div(col, a.by_group);
   const int qhead = kvh * G + (col - qi * G);
   // A request whose shared prefix was attended by span units (prefill jobs
   // only): fields 6 = first span partial slot + 1, 7 = the request's first
@@ -1182,8 +1201,10 @@ static int launch_merge_p(int64_t job_heads, int64_t max_columns, hipStream_t s,
                           int32_t num_kv_heads, int32_t group, int32_t col_tiles, const MergeArgs& a) {
   const int64_t groups = (max_columns + merge_columns<T, D, P> - 1) / merge_columns<T, D, P>;
   if (job_heads * groups > 0x7fffffffLL) return LVAMD_ERR_INVALID_ARGUMENT;
+  const FastDiv by_groups((int32_t)groups), by_heads(num_kv_heads);
   hipLaunchKernelGGL((paged_merge_kernel<T, D, P>), dim3((unsigned)(job_heads * groups)), dim3(64 * merge_waves(P)), 0,
-                     s, jobs, (int32_t)groups, num_kv_heads, group, col_tiles, a);
+                     s, jobs, (int32_t)groups, num_kv_heads, group, col_tiles, by_groups.magic, by_groups.shift,
+                     by_heads.magic, by_heads.shift, a);
   return launch_status();
 }
 
@@ -1197,7 +1218,7 @@ int launch_merge(const void* part_acc, const float* part_ml, void* out, int64_t 
   if (num_jobs < 0 || num_kv_heads <= 0 || group <= 0) return LVAMD_ERR_INVALID_ARGUMENT;
   if (num_jobs == 0) return LVAMD_OK;
   if (!part_acc || !part_ml || !out || !jobs) return LVAMD_ERR_INVALID_ARGUMENT;
-  MergeArgs a;
+  MergeArgs a{.by_group = FastDiv(group)};
   a.part_acc = part_acc;
   a.part_ml = part_ml;
   a.out = out;
@@ -1254,7 +1275,7 @@ extern "C" int lvamd_paged_decode(const void* q, int64_t q_token_stride, int64_t
                   (new_value_head_stride * es) % 16 != 0))
     return LVAMD_ERR_INVALID_ARGUMENT;
   if ((int64_t)waves_per_head * num_kv_heads > 0x7fffffffLL) return LVAMD_ERR_INVALID_ARGUMENT;
-  DecodeArgs a;
+  DecodeArgs a{.by_block = FastDiv(block_size), .by_group = FastDiv(group)};
   a.q = q;
   a.q_tok_stride = q_token_stride;
   a.q_head_stride = q_head_stride;
@@ -1276,22 +1297,22 @@ extern "C" int lvamd_paged_decode(const void* q, int64_t q_token_stride, int64_t
   a.num_kv_heads = num_kv_heads;
   a.group = group;
   a.block_size = block_size;
-  a.bs_shift = (block_size & (block_size - 1)) == 0 ? __builtin_ctz((unsigned)block_size) : -1;
   a.scale_log2 = scale * 1.4426950408889634f;
   const dim3 grid((unsigned)(waves_per_head / group_waves * num_kv_heads));
+  const FastDiv by_wg(waves_per_head / group_waves);
   hipStream_t s = static_cast<hipStream_t>(stream);
   return dispatch_decode(dtype, head_size, col_tiles, [&]<typename T, int D, int CTW>() -> int {
     if constexpr (CTW == 1) {
       constexpr int WG = split_waves<T, D>();
       if (group_waves == WG) {
         hipLaunchKernelGGL((paged_decode_kernel<T, D, CTW, WG>), grid, dim3(64 * WG), 0, s, wave_first, pieces,
-                           waves_per_head, a);
+                           waves_per_head, by_wg.magic, by_wg.shift, a);
         return launch_status();
       }
     }
     if (group_waves != 1) return LVAMD_ERR_UNSUPPORTED;
     hipLaunchKernelGGL((paged_decode_kernel<T, D, CTW, 1>), grid, dim3(64), 0, s, wave_first, pieces,
-                       waves_per_head, a);
+                       waves_per_head, by_wg.magic, by_wg.shift, a);
     return launch_status();
   });
 }
