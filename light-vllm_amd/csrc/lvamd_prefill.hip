@@ -141,7 +141,8 @@ struct PrefillArgs {
   float* part_ml;                        // [slots][Hkv][unit columns][2]: (max, sum)
   int32_t group;
   int32_t block_size;
-  int32_t bs_shift;
+  int32_t bs_shift;  // log2(block_size) when a power of two, else -1
+  FastDiv by_block, by_group;  // / block_size, / group
   float scale_log2;
 };
 
@@ -150,7 +151,7 @@ struct PrefillArgs {
 template <typename T, int D, int W, bool B16>
 __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W == 8 ? 4 : (D <= 128 ? 2 : 1)))) void paged_prefill_kernel(
     const int32_t* __restrict__ units,  // [n][LVAMD_PREFILL_FIELDS]
-    const int32_t num_kv_heads, const PrefillArgs a) {
+    const int32_t num_kv_heads, const uint32_t heads_magic, const int32_t heads_shift, const PrefillArgs a) {
   using P = PrefillShape<T, D, W>;
   constexpr int CPR = P::CPR, CG = P::CG, RB = P::RB, CT = P::CT, NCH = P::NCH, NT = P::NT;
   constexpr int KT = P::KT, KS = P::KS, GB = P::GROUP_BYTES;
@@ -170,8 +171,8 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W == 8 ?
   const int g = lane >> 4;
   const int Hkv = num_kv_heads;
   const int G = a.group;
-  const int unit = blockIdx.x / Hkv;
-  const int kvh = blockIdx.x - unit * Hkv;
+  const int unit = fast_div((int)blockIdx.x, heads_magic, heads_shift);
+  const int kvh = (int)blockIdx.x - unit * Hkv;
   // The unit record carries everything the unit needs, so the first tile's
   // loads depend on one load (the record) only: its request's fields (a span
   // unit, over keys every query of the span sees, reads as a linear request
@@ -186,7 +187,7 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W == 8 ?
   // Keys the unit needs: up to its last query's position, within the piece's
   // key range [key_begin, key_end) (key_begin a multiple of KT; key_end 0 =
   // no bound).  Tiles are numbered from position 0.
-  const int kneed = computed + (col_end - 1) / G + 1;
+  const int kneed = computed + fast_div(col_end - 1, a.by_group) + 1;
   const int kmax = key_end > 0 && key_end < kneed ? key_end : kneed;
   const int tile0 = key_begin / KT;
   const int ntiles = (kmax + KT - 1) / KT - tile0;  // tiles of this piece
@@ -213,7 +214,7 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W == 8 ?
   const int pool_end = knew != nullptr && computed < kmax ? computed : kmax;  // keys in the pool
   auto logical_block = [&](int pos) -> int {
     if constexpr (B16) return pos >> a.bs_shift;
-    return a.bs_shift >= 0 ? (pos >> a.bs_shift) : (pos / bs);
+    return fast_div(pos, a.by_block);
   };
   // The key whose block's table entry this lane needs: its row's, or (B16) its
   // row block's first.  Rows past the piece read its last key (masked).
@@ -335,7 +336,7 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W == 8 ?
     const int col = col0 + 16 * (CT * wave + ct) + l16;
     colok[ct] = col < col_end;
     const int colc = colok[ct] ? col : col_end - 1;
-    qi[ct] = colc / G;
+    qi[ct] = fast_div(colc, a.by_group);
     const int qhead = kvh * G + (colc - qi[ct] * G);
     const T* qrow = static_cast<const T*>(a.q) + (int64_t)(q_start + qi[ct]) * a.q_tok_stride +
                     (int64_t)qhead * a.q_head_stride;
@@ -347,11 +348,11 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W == 8 ?
   }
   // Keys this wave's columns can see at most (its last valid query).
   const int wave_col_last = col0 + 16 * CT * (wave + 1) - 1;
-  const int wave_kmax = computed + ((wave_col_last < col_end ? wave_col_last : col_end - 1) / G) + 1;
+  const int wave_kmax = computed + fast_div(wave_col_last < col_end ? wave_col_last : col_end - 1, a.by_group) + 1;
   const bool wave_active = col0 + 16 * CT * wave < col_end;
   // Tiles below this bound are visible to every column of the unit (for a
   // tree request only the computed prefix is).
-  const int full_tiles = (vis_off >= 0 ? computed : computed + col0 / G + 1) / KT;
+  const int full_tiles = (vis_off >= 0 ? computed : computed + fast_div(col0, a.by_group) + 1) / KT;
   const bool tree = vis_off >= 0;
   const float c_log2 = a.scale_log2;
   // A tree of at most 32 queries has one ancestor word per query: each
@@ -579,7 +580,7 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W == 8 ?
   // Pairs of tiles that no column masks, that hold none of this unit's own
   // tokens and that a tile follows; then the rest.
   int t = 0;
-  const int nfull = min((tree ? computed : computed + col0 / G) / KT - tile0, ntiles - 1) - 1;
+  const int nfull = min((tree ? computed : computed + fast_div(col0, a.by_group)) / KT - tile0, ntiles - 1) - 1;
   for (; t < nfull; t += 2) {
     step.template operator()<false>(t, klds0, vlds0, klds1, vlds1);
     step.template operator()<false>(t + 1, klds1, vlds1, klds0, vlds0);
@@ -620,10 +621,13 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W == 8 ?
 template <typename T, int D, int W>
 static int launch_prefill_w(dim3 grid, hipStream_t s, const int32_t* units, int32_t num_kv_heads, const PrefillArgs& a) {
   if constexpr (prefill_built(D, W)) {
+    const FastDiv by_heads(num_kv_heads);
     if (a.bs_shift >= 4) {
-      hipLaunchKernelGGL((paged_prefill_kernel<T, D, W, true>), grid, dim3(64 * W), 0, s, units, num_kv_heads, a);
+      hipLaunchKernelGGL((paged_prefill_kernel<T, D, W, true>), grid, dim3(64 * W), 0, s, units, num_kv_heads,
+                         by_heads.magic, by_heads.shift, a);
     } else {
-      hipLaunchKernelGGL((paged_prefill_kernel<T, D, W, false>), grid, dim3(64 * W), 0, s, units, num_kv_heads, a);
+      hipLaunchKernelGGL((paged_prefill_kernel<T, D, W, false>), grid, dim3(64 * W), 0, s, units, num_kv_heads,
+                         by_heads.magic, by_heads.shift, a);
     }
     return launch_status();
   }
@@ -755,7 +759,7 @@ extern "C" int lvamd_paged_prefill(const void* q, int64_t q_token_stride, int64_
                   (new_key_token_stride * es) % 16 != 0 || (new_key_head_stride * es) % 16 != 0 ||
                   (new_value_token_stride * es) % 16 != 0 || (new_value_head_stride * es) % 16 != 0))
     return LVAMD_ERR_INVALID_ARGUMENT;
-  PrefillArgs a;
+  PrefillArgs a{.by_block = FastDiv(block_size), .by_group = FastDiv(group)};
   a.q = q;
   a.q_tok_stride = q_token_stride;
   a.q_head_stride = q_head_stride;
