@@ -218,9 +218,8 @@ int lvamd_paged_decode_resident_waves(int32_t dtype, int32_t head_size, int32_t 
 int lvamd_paged_decode_tile_tokens(int32_t dtype, int32_t head_size, int32_t col_tiles);
 
 /*
- * Log-sum-exp merge of split-K partials into out, one wave per (job, kv head,
- * column), four columns per workgroup, over the first max_columns (1 to
- * 16 * col_tiles) columns of each job (the most any job has; the host knows
+ * Log-sum-exp merge of split-K partials into out, over the first max_columns
+ * (1 to 16 * col_tiles) columns of each job (the most any job has; the host knows
  * it); jobs [num_jobs][LVAMD_MERGE_FIELDS]; col_tiles (1 to 16) is
  * the number of 16-column tiles per partial slot the partials were written
  * with (the decode kernel's col_tiles, or prefill unit columns / 16).

@@ -24,7 +24,7 @@
 //     h * waves_per_head + w and walks its pieces (the parts of segments
 //     inside its share).  A piece covering a whole segment writes the output;
 //     the others write partials that the merge kernel combines by
-//     log-sum-exp, one wave per (segment, kv head, output column).  (Merging in
+//     log-sum-exp.  (Merging in
 //     the decode kernel, by the wave that completes a segment, put ~1000
 //     instructions of cold code in the kernel's tail: the instruction-cache
 //     misses cost more than a separate launch.)
