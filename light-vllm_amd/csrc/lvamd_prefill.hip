@@ -45,7 +45,6 @@
 
 #include "lvamd_common.h"
 
-
 namespace lvamd {
 
 namespace {
@@ -79,7 +78,6 @@ constexpr bool prefill_built(int d, int w) { return w == 4 || (w == 8 && d <= 12
 constexpr int prefill_key_tile(int d) { return d <= 128 ? kPrefillKeyTile : 32; }
 constexpr int prefill_unit_columns(int d) { return 16 * prefill_col_tiles_per_wave(d, 4) * 4; }
 static_assert(16 * 1 * 8 == 16 * 2 * 4, "both shapes cover the same unit columns");
-
 
 // LDS tile layout.  A K (or V) tile of KT rows is stored as CG column groups
 // (64 bytes = four 16-byte chunks of every row), group-major: byte
@@ -728,7 +726,7 @@ extern "C" int lvamd_paged_prefill_resident_units(int32_t dtype, int32_t head_si
 
 extern "C" int lvamd_paged_prefill_waves_built(int32_t dtype, int32_t head_size, int32_t waves) {
   if (!prefill_supported(dtype, head_size)) return 0;
-  return (waves == 4 || (waves == 8 && head_size <= 128 )) ? 1 : 0;
+  return (waves == 4 || (waves == 8 && head_size <= 128)) ? 1 : 0;
 }
 
 extern "C" int lvamd_paged_prefill(const void* q, int64_t q_token_stride, int64_t q_head_stride,
