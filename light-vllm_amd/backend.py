@@ -225,8 +225,8 @@ class HipPagedAttention:
         # step's (bound plan, output slab), bound at the shape's first layer.
         self._statics = backend.layer_statics(cache) if _raw_stream is not None else {}
         self._shape_bound: dict[tuple, tuple] = {}
+        self._rotary_bound: dict[tuple, tuple] = {}
         self._attend_tensors = backend._attend_tensors
-        self._attend_rotary = backend._attend_rotary
         self._attend_fn = backend._attend_fn
 
     @property
@@ -269,8 +269,10 @@ class HipPagedAttention:
                 status = self._attend_tensors(bound[0], static.k_pool, static.v_pool, bound[1] + index * bound[2],
                                               query, key, value, scale)
             else:
-                status = self._attend_rotary(bound[0], static.k_pool, static.v_pool, bound[1] + index * bound[2],
-                                             query, key, value, scale, rotary[0], rotary[1], bound[5], bound[6])
+                extra = self._rotary_bound.get(static.shape) or self._bind_rotary(static, bound[4])
+                status = self._backend._attend_rotary(bound[0], static.k_pool, static.v_pool,
+                                                      bound[1] + index * bound[2], query, key, value, scale,
+                                                      rotary[0], rotary[1], extra[0], extra[1])
             if status == 0:
                 return bound[3][index]
             if status != _NOT_FAST:
@@ -280,8 +282,7 @@ class HipPagedAttention:
     def _bind_shape(self, static) -> tuple:
         """The fast path's facts for the layers of one shape in this step:
         (the shape's facts for attend_tensors, the output slab's address,
-        its bytes per layer, the per-layer output views, the launch, the
-        rotary append's facts, the rotated-query buffer of a stream).
+        its bytes per layer, the per-layer output views, the launch).
 
         Outputs are views of one tensor per layer shape and step, made at the
         first layer of that shape (one allocation for the step's layers in
@@ -306,6 +307,18 @@ class HipPagedAttention:
             static.device_index, static.element_size, tokens, spec.num_query_heads, spec.num_kv_heads,
             spec.head_size, _raw_stream,
         )
+        bound = (facts, slab.data_ptr(), tokens * spec.num_query_heads * spec.head_size * static.element_size,
+                 views, launch)
+        self._shape_bound[static.shape] = bound
+        return bound
+
+    def _bind_rotary(self, static, launch) -> tuple:
+        """What attend_rotary needs beside _bind_shape's facts, made at the
+        first rotary layer of a shape so that other steps do not pay for it:
+        (the rotary append's facts, the rotated-query buffer of a stream)."""
+
+        spec = static.spec
+        tokens = self._plan.num_tokens
         rotated: dict[int, Tensor] = {}
 
         def rotated_queries(stream: int) -> int:
@@ -318,10 +331,9 @@ class HipPagedAttention:
                                                        dtype=static.dtype, device=static.device)
             return buffer.data_ptr()
 
-        bound = (facts, slab.data_ptr(), tokens * spec.num_query_heads * spec.head_size * static.element_size,
-                 views, launch, (self._backend._rotary_fn, self._plan.slots_ptr, launch.dtype), rotated_queries)
-        self._shape_bound[static.shape] = bound
-        return bound
+        extra = ((self._backend._rotary_fn, self._plan.slots_ptr, launch.dtype), rotated_queries)
+        self._rotary_bound[static.shape] = extra
+        return extra
 
     def _forward_general(self, layer_id: str, query: Tensor, key: Tensor, value: Tensor, *, scale: float,
                          rotary: tuple[Tensor, Tensor] | None) -> Tensor:
