@@ -234,6 +234,13 @@ int lvamd_paged_attention_merge(const void* part_acc, const float* part_ml,
                                 int32_t num_kv_heads, int32_t group, int32_t head_size, int32_t col_tiles,
                                 int32_t max_columns, int32_t dtype, lvamd_stream_t stream);
 
+/* Waves (1, 4 or 16) that share each column's partials in the merge of such a
+ * job list: num_partials over all jobs, merge_depth those of the deepest job
+ * (0 where not known); each wave requests 16 partials at a time.  Results do not
+ * depend on it beyond the order of the fp32 sums. */
+int lvamd_paged_merge_waves(int32_t dtype, int32_t head_size, int32_t num_jobs, int64_t num_partials,
+                            int32_t merge_depth, int32_t num_kv_heads, int32_t max_columns);
+
 /*
  * Chunked-prefill paged attention for query runs of more than one column
  * tile (prompt chunks, tree verification; bf16 / fp16, head sizes that are
@@ -291,6 +298,7 @@ typedef struct lvamd_attention_plan {
   int32_t num_jobs;
   int32_t merge_columns;
   int32_t group_waves; /* 1: stream-K; lvamd_paged_decode_split_waves: workgroup split */
+  int32_t merge_depth; /* partials of the deepest decode merge job (0: not known; picks the merge's shape only) */
   /* Prefill rows (num_units 0: none). */
   const int32_t* units;
   int32_t num_units;

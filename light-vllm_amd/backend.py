@@ -169,7 +169,7 @@ class _LayerLaunch:
             pieces=work.pieces_ptr, wave_first=work.wave_first_ptr, waves_per_head=work.waves_per_head,
             col_tiles=work.col_tiles, part_acc=part_acc, part_ml=part_ml, num_partial_slots=work.num_partial_slots,
             jobs=work.jobs_ptr, num_jobs=work.num_jobs, merge_columns=work.merge_columns,
-            group_waves=work.group_waves,
+            group_waves=work.group_waves, merge_depth=work.merge_depth,
             units=work.units_ptr, num_units=work.num_prefill_units, prefill_waves=work.prefill_waves,
             prefill_part_acc=pre_acc, prefill_part_ml=pre_ml,
             num_prefill_partial_slots=work.num_prefill_partial_slots, prefill_jobs=work.prefill_jobs_ptr,

@@ -27,8 +27,8 @@ extern "C" int lvamd_paged_attention(const lvamd_attention_plan* plan,
     if (status != LVAMD_OK) return status;
     if (p.num_jobs > 0) {
       status = launch_merge(p.part_acc, p.part_ml, out, out_token_stride, out_head_stride, p.jobs, p.num_jobs,
-                            p.num_partial_slots, p.num_kv_heads, p.group, p.head_size, p.col_tiles, p.merge_columns,
-                            p.dtype, static_cast<hipStream_t>(stream));
+                            p.num_partial_slots, p.merge_depth, p.num_kv_heads, p.group, p.head_size, p.col_tiles,
+                            p.merge_columns, p.dtype, static_cast<hipStream_t>(stream));
       if (status != LVAMD_OK) return status;
     }
   }
@@ -42,7 +42,7 @@ extern "C" int lvamd_paged_attention(const lvamd_attention_plan* plan,
     if (status != LVAMD_OK) return status;
     if (p.num_prefill_jobs > 0) {
       status = launch_merge(p.prefill_part_acc, p.prefill_part_ml, out, out_token_stride, out_head_stride,
-                            p.prefill_jobs, p.num_prefill_jobs, p.num_prefill_partial_slots, p.num_kv_heads, p.group,
+                            p.prefill_jobs, p.num_prefill_jobs, p.num_prefill_partial_slots, 0, p.num_kv_heads, p.group,
                             p.head_size, p.prefill_col_tiles, p.prefill_merge_columns, p.dtype,
                             static_cast<hipStream_t>(stream));
     }

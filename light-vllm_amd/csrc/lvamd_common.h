@@ -182,10 +182,10 @@ inline int launch_status() {
 }
 
 // lvamd_paged_attention_merge with the launch's partial count (all jobs; 0:
-// unknown), which picks the kernel's shape.
+// unknown) and its deepest job's (0: unknown), which pick the kernel's shape.
 int launch_merge(const void* part_acc, const float* part_ml, void* out, int64_t out_token_stride,
                  int64_t out_head_stride, const int32_t* jobs, int32_t num_jobs, int64_t num_partials,
-                 int32_t num_kv_heads, int32_t group, int32_t head_size, int32_t col_tiles, int32_t max_columns,
+                 int64_t merge_depth, int32_t num_kv_heads, int32_t group, int32_t head_size, int32_t col_tiles, int32_t max_columns,
                  int32_t dtype, hipStream_t s);
 
 }  // namespace lvamd

@@ -1208,9 +1208,25 @@ static int launch_merge_p(int64_t job_heads, int64_t max_columns, hipStream_t s,
   return launch_status();
 }
 
+// Waves that share a column's partials (the merge kernel's P).  What counts is
+// the deepest job, whose rounds of 16 P partials run one after the other while
+// the others are long done; without its depth, the mean of all jobs.  Merge
+// alone at P = 1 / 4 / 16, 4 kv heads, D = 128 bf16: 127 partials of one job
+// 15.9 / 6.1 / 5.5 us; 146 at most, in 64 jobs of 4.5 on average, 18.7 / 7.3 /
+// 8.1; 63 at most, in 32 jobs of 5.9, 8.9 / 4.5 / 5.1; 64 jobs of five 4.2 / 4.2 /
+// 6.8; 192 columns of 13 4.6 / 4.1 at P = 1 / 4.  Sixteen waves pay past 64
+// partials, and while their workgroups have a CU each (one fits a CU).
+constexpr int64_t kMergeFitWorkgroups = 256;
+static int merge_sharing(int64_t num_jobs, int64_t num_partials, int64_t merge_depth, int64_t workgroups) {
+  const int64_t mean = (num_partials + num_jobs - 1) / num_jobs;
+  const int64_t depth = merge_depth > 0 ? merge_depth : mean;
+  if (depth > 4 * kMergeRoundTrip && workgroups <= kMergeFitWorkgroups) return 16;
+  return depth > kMergeRoundTrip || mean > kMergeRoundTrip / 2 ? 4 : 1;
+}
+
 int launch_merge(const void* part_acc, const float* part_ml, void* out, int64_t out_token_stride,
                  int64_t out_head_stride, const int32_t* jobs, int32_t num_jobs, int64_t num_partials,
-                 int32_t num_kv_heads, int32_t group, int32_t head_size, int32_t col_tiles, int32_t max_columns,
+                 int64_t merge_depth, int32_t num_kv_heads, int32_t group, int32_t head_size, int32_t col_tiles, int32_t max_columns,
                  int32_t dtype, hipStream_t s) {
   if (dtype_size(dtype) == 0 || !head_size_supported(head_size) || col_tiles < 1 || col_tiles > 16)
     return LVAMD_ERR_UNSUPPORTED;
@@ -1226,15 +1242,12 @@ int launch_merge(const void* part_acc, const float* part_ml, void* out, int64_t 
   a.out_head_stride = out_head_stride;
   const int64_t job_heads = (int64_t)num_jobs * num_kv_heads;
   return dispatch_decode(dtype, head_size, 1, [&]<typename T, int D, int CTW>() -> int {
-    // Partials per job on average: one wave's requests grow with them (192
-    // columns of 13: 4.6 us at P = 1, 4.1 at P = 4; 1,792 columns of five:
-    // the same at both), and 129 partials take P = 4 three round trips
-    // (6.2 us against 4.6 at P = 16).
-    if (num_partials > 32 * (int64_t)num_jobs)
-      return launch_merge_p<T, D, 16>(job_heads, max_columns, s, jobs, num_kv_heads, group, col_tiles, a);
-    if (num_partials > 8 * (int64_t)num_jobs)
-      return launch_merge_p<T, D, 4>(job_heads, max_columns, s, jobs, num_kv_heads, group, col_tiles, a);
-    return launch_merge_p<T, D, 1>(job_heads, max_columns, s, jobs, num_kv_heads, group, col_tiles, a);
+    switch (merge_sharing(num_jobs, num_partials, merge_depth,
+                          job_heads * ((max_columns + merge_columns<T, D, 16> - 1) / merge_columns<T, D, 16>))) {
+      case 16: return launch_merge_p<T, D, 16>(job_heads, max_columns, s, jobs, num_kv_heads, group, col_tiles, a);
+      case 4: return launch_merge_p<T, D, 4>(job_heads, max_columns, s, jobs, num_kv_heads, group, col_tiles, a);
+      default: return launch_merge_p<T, D, 1>(job_heads, max_columns, s, jobs, num_kv_heads, group, col_tiles, a);
+    }
   });
 }
 
@@ -1360,11 +1373,21 @@ extern "C" int lvamd_paged_decode_resident_waves(int32_t dtype, int32_t head_siz
   });
 }
 
+extern "C" int lvamd_paged_merge_waves(int32_t dtype, int32_t head_size, int32_t num_jobs, int64_t num_partials,
+                                       int32_t merge_depth, int32_t num_kv_heads, int32_t max_columns) {
+  if (num_jobs < 1 || num_kv_heads < 1 || max_columns < 1) return LVAMD_ERR_INVALID_ARGUMENT;
+  return dispatch_decode(dtype, head_size, 1, [&]<typename T, int D, int CTW>() -> int {
+    constexpr int64_t C = merge_columns<T, D, 16>;
+    return merge_sharing(num_jobs, num_partials, merge_depth,
+                         (int64_t)num_jobs * num_kv_heads * ((max_columns + C - 1) / C));
+  });
+}
+
 extern "C" int lvamd_paged_attention_merge(const void* part_acc, const float* part_ml,
                                            void* out, int64_t out_token_stride, int64_t out_head_stride,
                                            const int32_t* jobs, int32_t num_jobs,
                                            int32_t num_kv_heads, int32_t group, int32_t head_size, int32_t col_tiles,
                                            int32_t max_columns, int32_t dtype, lvamd_stream_t stream) {
-  return launch_merge(part_acc, part_ml, out, out_token_stride, out_head_stride, jobs, num_jobs, 0, num_kv_heads,
+  return launch_merge(part_acc, part_ml, out, out_token_stride, out_head_stride, jobs, num_jobs, 0, 0, num_kv_heads,
                       group, head_size, col_tiles, max_columns, dtype, static_cast<hipStream_t>(stream));
 }

@@ -934,6 +934,7 @@ struct DecodeLists {
   int64_t waves = 0, per_wave = 0, merge_cols = 1;
   int64_t group_waves = 1;  // 1: stream-K; kSplitWaves: workgroup split
   int32_t slots = 0;
+  int32_t depth = 0;  // pieces of the deepest merge job
   void reset() {
     pieces.clear();
     first.clear();
@@ -941,7 +942,7 @@ struct DecodeLists {
     waves = per_wave = 0;
     merge_cols = 1;
     group_waves = 1;
-    slots = 0;
+    slots = depth = 0;
   }
 };
 
@@ -977,9 +978,13 @@ struct DecodeParams {
 constexpr int64_t kSplitMergeTiles = 3;
 constexpr int64_t kMergePiecesMax = 48;
 // With the merge's sixteen-wave shape (merge_pieces above kMergePiecesMax) a
-// lone long sequence is spread over up to that many shares: one tile each up
-// to kOneTilePieces of them, two or more past that.  Per layer at 28 / 4
-// heads, D 128, bf16: one sequence of 8,112 tokens (254 tiles) 23.3 us in 43
+// long sequence is spread over up to that many shares, alone or beside
+// others: one tile each up to kOneTilePieces of them, two or more past that.
+// The merge's shape follows the deepest segment (DecodeLists::depth).  Per
+// layer at 28 / 4 heads, D 128, bf16, with at most 48 / at most 256 pieces:
+// 32,701 tokens beside 63 of 300 52.7 / 34.5 us, 6,000 beside 15 of 300 18.9 /
+// 17.1, 4,000 beside 31 of 200 17.6 / 17.8, 16,000 beside 127 of 1,000 58 /
+// 58.  One sequence of 8,112 tokens (254 tiles) 23.3 us in 43
 // shares of six tiles, 17.9 in 86 of three, 16.9 in 127 of two, 19.4 in 254
 // of one; 32,701 tokens 58 us in 47 shares, 32.4 in 147, 30.6 in 205; 2,048
 // tokens 13.2 us in 33 shares of two, 12.8 in 64 of one.
@@ -1089,6 +1094,7 @@ void build_decode(const Requests& q, const int32_t* ids, int64_t nflat, const De
     if (multi && x.lo == sg.start) {
       const int32_t job[kMergeFields] = {sg.req, sg.group, out.slots, seg_pieces[(size_t)x.seg], m[4], m[3], 0, 0};
       out.jobs.insert(out.jobs.end(), job, job + kMergeFields);
+      out.depth = std::max(out.depth, job[3]);
       // The merge grid covers the most columns any job has.
       out.merge_cols = std::max(out.merge_cols, std::min(per_slot, (int64_t)m[3] * d.group - sg.group * per_slot));
     }
@@ -1543,8 +1549,8 @@ PyObject* decode_result(const DecodeLists& d) {
   PyObject* a = to_bytearray(d.pieces);
   PyObject* b = to_bytearray(d.first);
   PyObject* c = to_bytearray(d.jobs);
-  PyObject* result = (a && b && c) ? Py_BuildValue("(OOOLLiLL)", a, b, c, (long long)d.waves, (long long)d.per_wave,
-                                                   d.slots, (long long)d.merge_cols, (long long)d.group_waves)
+  PyObject* result = (a && b && c) ? Py_BuildValue("(OOOLLiLLi)", a, b, c, (long long)d.waves, (long long)d.per_wave,
+                                                   d.slots, (long long)d.merge_cols, (long long)d.group_waves, d.depth)
                                    : nullptr;
   Py_XDECREF(a);
   Py_XDECREF(b);
@@ -1587,7 +1593,7 @@ bool requests_of(const Buf& meta, Requests* q, const char* name) {
 //             max_units_per_wave (0 = none), unit_tokens, split_groups, split_waves)
 //   -> (pieces i32 [n, 16], wave_first i32 [W + 1], jobs i32 [m, 8],
 //       W, largest share, partial slots, most columns of a merge job,
-//       waves per workgroup)
+//       waves per workgroup, pieces of the deepest merge job)
 // split_groups: resident workgroups of the workgroup-split kernel (0: never
 // split in workgroups) and split_waves its waves per workgroup.
 PyObject* decode_work(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
@@ -1785,7 +1791,7 @@ const char* plan_layer(const Requests& q, const int32_t* ids, int64_t nflat, con
 //    decode partial slots, decode merge jobs, decode merge columns,
 //    prefill units, prefill merge jobs, prefill partial slots,
 //    prefill merge columns, pieces, wave_first, jobs, units, prefill jobs,
-//    decode pieces, decode waves per workgroup)
+//    decode pieces, decode waves per workgroup, pieces of the deepest decode merge job)
 // with the five offsets -1 for an absent list.
 // ---------------------------------------------------------------------------
 std::vector<LayerPlan> g_layer_plans;
@@ -1892,7 +1898,7 @@ PyObject* plan_step(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     const DecodeLists& d = plan.dec;
     const PrefillLists& p = plan.pre;
     PyObject* one = Py_BuildValue(
-        "(LLLLLLLLLLLLLLLLLL)", (long long)plan.ctw, (long long)plan.waves, (long long)(plan.has_dec ? d.waves : 0),
+        "(LLLLLLLLLLLLLLLLLLL)", (long long)plan.ctw, (long long)plan.waves, (long long)(plan.has_dec ? d.waves : 0),
         (long long)(plan.has_dec ? d.per_wave : 0), (long long)(plan.has_dec ? d.slots : 0),
         (long long)(plan.has_dec ? (int64_t)d.jobs.size() / kMergeFields : 0),
         (long long)(plan.has_dec ? d.merge_cols : 1),
@@ -1901,7 +1907,7 @@ PyObject* plan_step(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
         (long long)(plan.has_pre ? p.merge_cols : 1), (long long)o.pieces, (long long)o.first, (long long)o.jobs,
         (long long)o.units, (long long)o.pjobs,
         (long long)(plan.has_dec ? (int64_t)d.pieces.size() / kPieceFields : 0),
-        (long long)(plan.has_dec ? d.group_waves : 1));
+        (long long)(plan.has_dec ? d.group_waves : 1), (long long)(plan.has_dec ? d.depth : 0));
     if (one == nullptr) {
       Py_DECREF(shapes);
       return nullptr;

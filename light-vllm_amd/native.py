@@ -67,6 +67,7 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
         ctypes.c_int,
         [_p, _p, _p, _i64, _i64, _p, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _p],
     ),
+    "lvamd_paged_merge_waves": (ctypes.c_int, [_i32, _i32, _i32, _i64, _i32, _i32, _i32]),
     "lvamd_paged_prefill": (
         ctypes.c_int,
         [_p, _i64, _i64, _p, _i64, _i64, _p, _i64, _i64, _p, _p, _p, _i64, _i64, _p, _p, _p, _i32, _p, _p, _i64,
@@ -115,6 +116,7 @@ class AttentionPlan(ctypes.Structure):
         ("pieces", _p), ("wave_first", _p), ("waves_per_head", _i32), ("col_tiles", _i32),
         ("part_acc", _p), ("part_ml", _p), ("num_partial_slots", _i64),
         ("jobs", _p), ("num_jobs", _i32), ("merge_columns", _i32), ("group_waves", _i32),
+        ("merge_depth", _i32),
         ("units", _p), ("num_units", _i32), ("prefill_waves", _i32),
         ("prefill_part_acc", _p), ("prefill_part_ml", _p), ("num_prefill_partial_slots", _i64),
         ("prefill_jobs", _p), ("num_prefill_jobs", _i32), ("prefill_merge_columns", _i32),

@@ -46,8 +46,9 @@ DECODE_MAX_COLUMNS = 16
 # longer set the step's pace); steps that fill the resident waves are not
 # affected.
 DECODE_MIN_UNITS_PER_WAVE = 1
-# Most pieces of one decode segment: the merge's sixteen-wave shape combines
-# 256 partials in one round trip.
+# Most pieces of one decode segment, in any step: the merge's sixteen-wave
+# shape combines 256 partials in one round trip, its four-wave shape (deep
+# segments in steps of many columns) in four.
 DECODE_MERGE_PIECES = 256
 # Smallest key range (in prefill key tiles) the planner gives one prefill
 # workgroup when it splits units to fill the GPU.
@@ -212,7 +213,7 @@ class DecodeWork:
     __slots__ = ("pieces_host", "wave_first_host", "jobs_host", "units_host", "prefill_jobs_host",
                  "waves_per_head", "num_jobs", "num_partial_slots", "units_per_wave", "col_tiles", "group_waves",
                  "num_prefill_units", "num_prefill_jobs", "num_prefill_partial_slots", "prefill_waves",
-                 "merge_columns", "prefill_merge_columns", "pieces_ptr", "wave_first_ptr", "jobs_ptr",
+                 "merge_columns", "prefill_merge_columns", "merge_depth", "pieces_ptr", "wave_first_ptr", "jobs_ptr",
                  "units_ptr", "prefill_jobs_ptr", "_staged")
 
     def __init__(self, *, col_tiles: int, prefill_waves: int) -> None:
@@ -226,6 +227,7 @@ class DecodeWork:
         self.waves_per_head = self.num_jobs = self.num_partial_slots = self.units_per_wave = 0
         self.num_prefill_units = self.num_prefill_jobs = self.num_prefill_partial_slots = 0
         self.merge_columns = self.prefill_merge_columns = 1  # most columns any merge job has
+        self.merge_depth = 0  # partials of the deepest decode merge job
         self.pieces_ptr = self.wave_first_ptr = self.jobs_ptr = self.units_ptr = self.prefill_jobs_ptr = None
         self._staged = None  # (uploaded blob, {list name: (offset, rows, fields)}) of a fused plan
 
@@ -235,9 +237,9 @@ class DecodeWork:
         uploaded step buffer): counts from ``row``, lists only on the device."""
 
         (ctw, waves, wph, per_wave, slots, njobs, mcols, nunits, npjobs, pslots, pmcols,
-         o_pieces, o_first, o_jobs, o_units, o_pjobs, npieces, group_waves) = row
+         o_pieces, o_first, o_jobs, o_units, o_pjobs, npieces, group_waves, depth) = row
         work = cls(col_tiles=ctw, prefill_waves=waves)
-        work.group_waves = group_waves
+        work.group_waves, work.merge_depth = group_waves, depth
         work.waves_per_head, work.units_per_wave, work.num_partial_slots = wph, per_wave, slots
         work.num_jobs, work.merge_columns = njobs, mcols
         work.num_prefill_units, work.num_prefill_jobs = nunits, npjobs
@@ -630,8 +632,8 @@ def _fill_work(work: DecodeWork, dec, pre) -> None:
     """Store the native planner's decode and prefill results in ``work``."""
 
     if dec is not None:
-        pieces, first, jobs, waves, per_wave, slots, merge_cols, group_waves = dec
-        work.group_waves = int(group_waves)
+        pieces, first, jobs, waves, per_wave, slots, merge_cols, group_waves, depth = dec
+        work.group_waves, work.merge_depth = int(group_waves), int(depth)
         work.pieces_host = _as_i32(pieces).reshape(-1, PIECE_FIELDS)
         work.wave_first_host = _as_i32(first)
         work.jobs_host = _as_i32(jobs).reshape(-1, MERGE_FIELDS)

@@ -8,7 +8,8 @@ import pytest
 import torch
 
 import light_vllm_amd as lv
-from light_vllm_amd.plan import DECODE_MERGE_PIECES, KERNEL_FACTS, StepPlan
+from light_vllm_amd import native
+from light_vllm_amd.plan import DECODE_MERGE_PIECES, KERNEL_FACTS, LayerShapes, StepPlan
 
 # 4 kv heads, 16-token blocks, 1024 resident waves of 32-token tiles.
 FACTS = (7, 4, 16, 0, 0, 0, 0, 0, 1, 0, 1024, 32, 0, 0, 0, 0, 0, 16, 1, 4, 0, 0, 0, 0, 8)
@@ -37,3 +38,33 @@ def test_kernel_facts_may_leave_out_only_the_optional_ones() -> None:
     assert _work(5000).pieces.tolist() == _work(5000, 0).pieces.tolist()
     with pytest.raises(ValueError):
         _work(5000, 0, 0)
+
+
+# (lengths, bound on the merge's rounds of its deepest job): one deep segment
+# beside many shallow ones, where the mean says nothing about the deepest.
+@pytest.mark.parametrize("lens, rounds", (
+    ([32702] + [300] * 63, 3), ([32702] + [300] * 31, 1), ([32702] * 2 + [400] * 30, 1), ([4000] + [200] * 31, 1),
+    ([8111] + [64] * 31, 1), ([16000] + [1000] * 127, 4), ([65536], 1), ([1500] * 64, 1), ([300], 1)))
+def test_merge_rounds_follow_the_deepest_job(lens, rounds) -> None:
+    blocks = [-(-n // 16) for n in lens]
+    tables = tuple(tuple(range(sum(blocks[:i]), sum(blocks[:i + 1]))) for i in range(len(lens)))
+    md = lv.PagedAttentionMetadata(block_tables=tables, num_computed_tokens=tuple(n - 1 for n in lens),
+                                   query_layouts=(lv.linear_query_layout(1),) * len(lens))
+    key = FACTS + (DECODE_MERGE_PIECES,)
+    plan = lambda **kw: StepPlan(md, block_size=16, device=torch.device("cpu"), **kw).layer_work(key)  # noqa: E731
+    work, fused = plan(), plan(num_blocks=sum(blocks), shapes=LayerShapes([key]))
+    depth = int(work.jobs.numpy()[:, 3].max())
+    assert work.merge_depth == fused.merge_depth == depth <= DECODE_MERGE_PIECES
+    waves = native.load().lvamd_paged_merge_waves(2, 128, work.num_jobs, work.num_partial_slots, depth, 4,
+                                                  work.merge_columns)
+    assert waves in (1, 4, 16) and -(-depth // (16 * waves)) <= rounds
+
+
+def test_merge_waves_by_depth_mean_and_columns() -> None:
+    waves = lambda jobs, partials, depth, heads=4, columns=7, d=128: (  # noqa: E731
+        native.load().lvamd_paged_merge_waves(2, d, jobs, partials, depth, heads, columns))
+    assert [waves(64, 312, n) for n in (9, 16, 17, 64, 65, 256)] == [1, 1, 4, 4, 4, 4]
+    assert [waves(32, 200, n) for n in (16, 17, 64, 65, 256)] == [1, 4, 4, 16, 16]  # 256 workgroups of two per head
+    assert [waves(32, n, 0) for n in (256, 257, 2048, 2049)] == [1, 4, 4, 16]  # the mean where no depth is known
+    assert waves(1, 16, 16, 4, 7) == 4 and waves(1, 8, 8) == 1
+    assert waves(0, 0, 0) == -1 and waves(1, 2, 2, d=72) == -2
