@@ -236,8 +236,9 @@ int lvamd_paged_attention_merge(const void* part_acc, const float* part_ml,
 
 /* Waves (1, 4 or 16) that share each column's partials in the merge of such a
  * job list: num_partials over all jobs, merge_depth those of the deepest job
- * (0 where not known); each wave requests 16 partials at a time.  Results do not
- * depend on it beyond the order of the fp32 sums. */
+ * (0 where not known; lvamd_paged_attention_merge knows neither and goes by the
+ * sizes); each wave requests 16 partials at a time.  Results do not depend on
+ * it beyond the order of the fp32 sums. */
 int lvamd_paged_merge_waves(int32_t dtype, int32_t head_size, int32_t num_jobs, int64_t num_partials,
                             int32_t merge_depth, int32_t num_kv_heads, int32_t max_columns);
 

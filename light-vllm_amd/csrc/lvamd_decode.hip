@@ -1217,7 +1217,17 @@ static int launch_merge_p(int64_t job_heads, int64_t max_columns, hipStream_t s,
 // 6.8; 192 columns of 13 4.6 / 4.1 at P = 1 / 4.  Sixteen waves pay past 64
 // partials, and while their workgroups have a CU each (one fits a CU).
 constexpr int64_t kMergeFitWorkgroups = 256;
+constexpr int64_t kMergeFewWorkgroups = 32;  // four jobs of four heads and eight columns at D = 128
 static int merge_sharing(int64_t num_jobs, int64_t num_partials, int64_t merge_depth, int64_t workgroups) {
+  if (merge_depth <= 0 && num_partials <= 0) {
+    // A bare job list may be deep: the sizes decide.  (A list of deep
+    // segments only has few columns: sixteen waves, 5.5 us against 15.9 at P = 1
+    // for 127 partials of one job, 4.8 against 4.6 for 19; up to 1,024
+    // workgroups four waves cost short jobs nothing, 128 jobs of three
+    // 4.4 / 4.5; beyond, the extra waves do: 57,344 columns of two 30.3 / 11.1.)
+    if (workgroups <= kMergeFewWorkgroups) return 16;
+    return workgroups <= 4 * kMergeFitWorkgroups ? 4 : 1;
+  }
   const int64_t mean = (num_partials + num_jobs - 1) / num_jobs;
   const int64_t depth = merge_depth > 0 ? merge_depth : mean;
   if (depth > 4 * kMergeRoundTrip && workgroups <= kMergeFitWorkgroups) return 16;

@@ -67,4 +67,6 @@ def test_merge_waves_by_depth_mean_and_columns() -> None:
     assert [waves(32, 200, n) for n in (16, 17, 64, 65, 256)] == [1, 4, 4, 16, 16]  # 256 workgroups of two per head
     assert [waves(32, n, 0) for n in (256, 257, 2048, 2049)] == [1, 4, 4, 16]  # the mean where no depth is known
     assert waves(1, 16, 16, 4, 7) == 4 and waves(1, 8, 8) == 1
+    # A bare job list (neither known): by its workgroups.
+    assert [waves(n, 0, 0) for n in (1, 4, 5, 128, 129)] == [16, 16, 4, 4, 1]
     assert waves(0, 0, 0) == -1 and waves(1, 2, 2, d=72) == -2

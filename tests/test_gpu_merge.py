@@ -65,3 +65,37 @@ def test_one_deep_job_among_shallow_ones(computed, hq, hkv, d, dtype, shape, rou
     err = np.abs(out.float().cpu().numpy() - dense_oracle_attention(step, step.layer_ids[0]))
     max_tol, mean_tol = tolerances(DTYPES[dtype])
     assert err.max() <= max_tol and err.mean() <= mean_tol
+
+
+@pytest.mark.parametrize("jobs, waves", ((1, 16), (10, 16), (11, 4), (341, 4), (342, 1)))
+@pytest.mark.parametrize("d, dtype", ((128, "bf16"), (48, "fp16"), (112, "fp32")))
+def test_bare_job_list(jobs, waves, d, dtype) -> None:
+    """The separate merge entry on made-up partials: its first job deeper than
+    a round trip of every shape, one partial empty.  A result is the weighted
+    mean of rows already in the pool's type, so it may differ by its own
+    rounding and by fp32 sums of 300 terms."""
+    hkv, group = 3, 2
+    assert native.load().lvamd_paged_merge_waves(dtype_code(DTYPES[dtype]), d, jobs, 0, 0, hkv, group) == waves
+    depth = [300] + [1 + i % 5 for i in range(jobs - 1)]
+    rng = np.random.default_rng(jobs)
+    start = np.cumsum([0] + depth)
+    records = torch.tensor([[i, 0, start[i], n, i, 1, 0, 0] for i, n in enumerate(depth)], dtype=torch.int32).cuda()
+    acc = torch.from_numpy(rng.standard_normal((start[-1], hkv, 16, d), dtype=np.float32)).to(DTYPES[dtype]).cuda()
+    pairs = np.stack((rng.uniform(-6, 6, (start[-1], hkv, 16)), rng.uniform(1, 9, (start[-1], hkv, 16))), -1)
+    pairs[7] = (-np.inf, 0.0)
+    ml = torch.from_numpy(pairs.astype(np.float32)).cuda()
+    out = torch.empty((jobs, hkv * group, d), dtype=DTYPES[dtype], device="cuda:0")
+    native.check(native.load().lvamd_paged_attention_merge(
+        acc.data_ptr(), ml.data_ptr(), out.data_ptr(), out.stride(0), out.stride(1), records.data_ptr(), jobs, hkv, group,
+        d, 1, group, dtype_code(DTYPES[dtype]), torch.cuda.current_stream().cuda_stream), "lvamd_paged_attention_merge")
+    rows, stats = acc.double().cpu().numpy()[:, :, :group], ml.double().cpu().numpy()[:, :, :group]
+    unit = {"bf16": 2.0 ** -8, "fp16": 2.0 ** -11, "fp32": 2.0 ** -24}[dtype]  # 2 ** -p: p significant bits, to nearest
+    for i in range(jobs):
+        m = stats[start[i]:start[i + 1]]
+        weight = np.exp2(m[..., 0] - m[..., 0].max(0)) * m[..., 1]
+        part = rows[start[i]:start[i + 1]] * weight[..., None]
+        want = (part.sum(0) / weight.sum(0)[..., None]).reshape(hkv * group, d)
+        size = (np.abs(part).sum(0) / weight.sum(0)[..., None]).reshape(hkv * group, d)
+        bound = unit * np.abs(want) + 400 * 2.0 ** -24 * size + 2.0 ** -24  # (last: fp16 below its normal range)
+        excess = (np.abs(out[i].double().cpu().numpy() - want) - bound).max()
+        assert excess <= 0, i
