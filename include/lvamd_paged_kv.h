@@ -349,7 +349,9 @@ int lvamd_paged_prefill_key_tokens(int32_t dtype, int32_t head_size);
 
 /* Prefill workgroups of the given shape (waves 4 or 8) the current device
  * holds at once for this dtype and head size: the planner splits units' key
- * ranges to fill them.  Needs a GPU. */
+ * ranges to fill them.  (Of the kernel for block sizes that are powers of two
+ * from 16; the one for other block sizes takes no more registers, so at least as
+ * many of it are.)  Needs a GPU. */
 int lvamd_paged_prefill_resident_units(int32_t dtype, int32_t head_size, int32_t waves);
 
 /* 1 when the prefill kernel is built with that many waves per workgroup for

@@ -247,7 +247,13 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W == 8 ?
   // block wholly in the pool or wholly in the step's input (nonnegative
   // strides that fit 32 bits) takes a scalar base and a fixed lane offset; the
   // block that holds the border, or the piece's end, an address per lane.
+  // (Without B16 at D = 128 the input's rows too: the two lane offsets are the
+  // registers that the eight-wave kernel has not got, 7 spills and 32 bytes of
+  // scratch with them.  Without them, at blocks of 12: 32 trees 27.1 -> 26.6 us a
+  // layer, four ragged prompts 27.6 -> 27.2, 1,024 over 8,000 on four waves
+  // 166.6 -> 164.2; at D = 32 and 64 they gain 1-2%.)
   constexpr bool kWhole = 4 * CG == CPR;
+  constexpr bool kFreshBlocks = B16 || D != 128;
   const int lane_chunk = kWhole ? lchunk * 8 : 0;
   const uint32_t pool_voff = (uint32_t)((lane >> 2) * (int)row_elems + lane_chunk) * 2u;
   const bool fresh_rows = knew != nullptr && a.kn_tok_stride >= 0 && a.kn_tok_stride < (1 << 24) &&
@@ -266,7 +272,7 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W == 8 ?
         return {(gptr<const char>)(kbase + off) + pool_voff, (gptr<const char>)(vbase + off) + pool_voff};
       }
     }
-    if (fresh_rows && p0 >= computed && p0 + 16 <= kmax) {
+    if (kFreshBlocks && fresh_rows && p0 >= computed && p0 + 16 <= kmax) {
       const int64_t row = q_start + p0 - computed;
       return {(gptr<const char>)(knew + row * a.kn_tok_stride) + kn_voff,
               (gptr<const char>)(vnew + row * a.vn_tok_stride) + vn_voff};

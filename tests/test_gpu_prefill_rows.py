@@ -1,8 +1,9 @@
 """GPU test: the prefill kernel's ways to address the step's K/V rows.  Row
 blocks of 16 in the step's input take a scalar base up to token strides of
-2**24 elements and an address per lane from there on; both, and rows shared by
-all tokens (stride 0), equal the same rows laid out contiguously bit for bit,
-in the outputs and in the pool."""
+2**24 elements and an address per lane from there on (always at D = 128 with
+block sizes other than powers of two from 16); both, and rows shared by all
+tokens (stride 0), equal the same rows laid out contiguously bit for bit, in
+the outputs and in the pool."""
 
 from __future__ import annotations
 
@@ -17,9 +18,9 @@ if not torch.cuda.is_available():
     pytest.skip("needs an MI355X GPU", allow_module_level=True)
 
 
-def _run(bs: int, queries: int, stride: int | None, spread: bool):
+def _run(d: int, bs: int, queries: int, stride: int | None, spread: bool):
     # 16 cached tokens: the chunk's first row block lies wholly in the input, its last one is cut short.
-    step = make_step(hq=4, hkv=2, d=64, bs=bs, dtype=torch.bfloat16, computed=[40, 16],
+    step = make_step(hq=4, hkv=2, d=d, bs=bs, dtype=torch.bfloat16, computed=[40, 16],
                      layouts=[(-1,), tuple(range(-1, queries - 1))], seed=bs)
     key, value = step.key, step.value
     if stride == 0:
@@ -27,7 +28,7 @@ def _run(bs: int, queries: int, stride: int | None, spread: bool):
         if not spread:
             key, value = key.contiguous(), value.contiguous()
     elif spread:
-        key, value = (torch.empty_strided(t.shape, (stride, 64, 1), dtype=t.dtype, device=t.device).copy_(t)
+        key, value = (torch.empty_strided(t.shape, (stride, d, 1), dtype=t.dtype, device=t.device).copy_(t)
                       for t in (key, value))
     layer = step.cache.layer("layer0")
     held = torch.zeros(layer.keys.shape[:2], dtype=torch.bool)  # the cached rows; every other row starts at 0
@@ -42,10 +43,10 @@ def _run(bs: int, queries: int, stride: int | None, spread: bool):
     return out, layer.keys, layer.values
 
 
+@pytest.mark.parametrize("d", (64, 128))
 @pytest.mark.parametrize("bs", (16, 32, 12))
-@pytest.mark.parametrize("queries,stride", ((40, 0), (40, 136), (24, (1 << 24) - 8), (24, 1 << 24)))
-def test_row_strides_of_the_step_equal_contiguous_rows(bs, queries, stride) -> None:
-    print(f"prefill rows bs={bs} queries={queries} stride={stride}", flush=True)
-    got, want = (_run(bs, queries, stride, spread) for spread in (True, False))
+@pytest.mark.parametrize("queries,stride", ((40, 0), (40, 264), (24, (1 << 24) - 8), (24, 1 << 24)))
+def test_row_strides_of_the_step_equal_contiguous_rows(d, bs, queries, stride) -> None:
+    got, want = (_run(d, bs, queries, stride, spread) for spread in (True, False))
     for a, b in zip(got, want):
         assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
