@@ -22,6 +22,18 @@ def _rows(tokens: int, d: int, dtype, strided: bool):
     return (rows[:, :d], rows[:, d:]) if strided else (rows[:, :d].contiguous(), rows[:, d:].contiguous())
 
 
+def _count_general(ctx) -> list[str]:
+    """The layers that take the general path from here on."""
+    taken, forward = [], ctx._forward_general
+
+    def counted(layer_id, *args, **kw):
+        taken.append(layer_id)
+        return forward(layer_id, *args, **kw)
+
+    ctx._forward_general = counted
+    return taken
+
+
 def _run(case, general: bool, views: bool, strided: bool, streams: bool = False):
     step = make_step(**case)
     pools = [t for lid in step.layer_ids for t in (step.cache.layer(lid).keys, step.cache.layer(lid).values)]
@@ -32,6 +44,7 @@ def _run(case, general: bool, views: bool, strided: bool, streams: bool = False)
     for t in pools:
         t[~held.cuda()] = 0
     ctx = lv.HipPagedAttentionBackend().create(step.cache, step.metadata)
+    generals = _count_general(ctx)
     if general:
         ctx._statics = {}  # no native call: every layer takes the general path
     tokens, d = step.query.shape[0], case["d"]
@@ -49,6 +62,7 @@ def _run(case, general: bool, views: bool, strided: bool, streams: bool = False)
             outs.append(ctx.forward(lid, q, k, v, scale=step.scale, rotary=rotary))
         torch.cuda.current_stream().wait_stream(side)  # (the split-K workspace is the stream's)
     torch.cuda.synchronize()
+    assert len(generals) == (len(step.layer_ids) if general else 0)
     return outs, pools
 
 
@@ -65,19 +79,26 @@ def test_native_rotary_call_equals_the_general_path(dtype, d, bs, views, strided
 
 
 def test_other_rotary_arguments_take_the_general_path() -> None:
-    case = dict(hq=4, hkv=2, d=64, bs=16, dtype=torch.bfloat16, computed=[40], layouts=[(-1,)], seed=3, num_layers=5)
+    case = dict(hq=4, hkv=2, d=64, bs=16, dtype=torch.bfloat16, computed=[40], layouts=[(-1,)], seed=3, num_layers=6)
     step = make_step(**case)
-    for own, first in zip(*((step.cache.layer(lid).keys, step.cache.layer(lid).values) for lid in ("layer1", "layer0"))):
-        own.copy_(first)
+    first = step.cache.layer("layer0")
+    for layer in (step.cache.layer("layer1"), step.cache.layer("layer5")):
+        layer.keys.copy_(first.keys)
+        layer.values.copy_(first.values)
     ctx = lv.HipPagedAttentionBackend().create(step.cache, step.metadata)
     cos, sin = _rows(1, 64, torch.bfloat16, False)
+    generals = _count_general(ctx)
     call = lambda i, q, r: ctx.forward(f"layer{i}", q, step.key, step.value, scale=step.scale, rotary=r)  # noqa: E731
     first = call(0, step.query, (cos, sin))
     shifted = torch.empty(4 * 64 + 1, dtype=torch.bfloat16, device="cuda:0")[1:].view(1, 4, 64).copy_(step.query)
-    assert torch.equal(call(1, shifted, [cos, sin]), first)
+    assert generals == []
+    assert torch.equal(call(1, step.query, [cos, sin]), first)
+    assert torch.equal(call(5, shifted, (cos, sin)), first)
+    assert generals == ["layer1", "layer5"]
     with pytest.raises(lv.KVCacheError, match="rotary cosines must have shape"):
         call(2, step.query, (cos[:, :32], sin))
     with pytest.raises(lv.KVCacheError, match="rotary sines dtype and device"):
         call(3, step.query, (cos, sin.float()))
     with pytest.raises(lv.KVCacheError, match="rotary cosines must have shape"):
         call(4, step.query, (None, sin))
+    assert generals == ["layer1", "layer5", "layer2", "layer3", "layer4"]
