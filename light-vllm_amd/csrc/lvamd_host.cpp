@@ -1515,15 +1515,20 @@ int64_t choose_col_tiles(const Requests& q, int64_t group, int64_t max_cols, int
 // has few key tiles (latency counts), else 4 waves of two column tiles (each
 // LDS read feeds two MFMAs).  With split-K the line is kWideShareTiles key
 // tiles per resident 8-wave workgroup; without (no resident count) it is a
-// mean of wide_max_tiles per unit.  Measured per step of 2-8 layers (28 / 4
-// heads, D 128 unless named), 8 waves / 4 waves, by tiles per slot: 0.8 (four
-// trees) 128 / 136 us, 3 (32 trees) 226 / 223, 4.5 (16 chunks of 64 over 500)
-// 248 / 250, 5.2 (1,000 over 1,000, D 64) 166 / 179, 7.3 (16 ragged prompts,
-// D 64) 122 / 145, 7.5 (16 of 300 over 300, 12 / 2 heads) 346 / 354, 7.2 (two
-// of 1,000) 359 / 349, 8.0 (eight of 512) 334 / 323, 11.5 (four of 200 over
-// 2K) 455 / 433, 15 (512 over 4K) 504 / 474, 57 (4,096) 596 / 545, 114 (two of
-// 512 over 16K) 1220 / 1116, 210 (2,048 over 14K) 1035 / 936; the other way
-// only 14.7 (eight of 128 over 2K) 520 / 539.
+// mean of wide_max_tiles per unit.  Measured per layer (28 / 4 heads, D 128
+// unless named), 8 waves / 4 waves in us, by tiles per workgroup:
+//   for the line: 0.8 (four trees) 15.5 / 16.6, 4.5 (16 chunks of 64 over 500)
+//   33.0 / 33.2, 4.6 (eight of 200 over 1,000, 8 / 8 heads, D 64) 23.5 / 24.9, 5.2
+//   (1,000 over 1,000, D 64) 25.4 / 29.8, 7.3 (16 ragged prompts, D 64) 32.0 /
+//   36.5, 7.5 (16 of 300 over 300, 12 / 2 heads) 44.9 / 45.8; 8.0 (eight of 512)
+//   44.8 / 42.9, 8.4 (16 of 64 over 1,000) 41.1 / 38.4, 11.8 (four of 200 over
+//   2K) 61.9 / 58.2, 14.7 (eight of 128 over 2K) 66.0 / 63.2, 57 (4,096) 151 /
+//   140, 110 (512 over 32K) 345 / 307, 210 (2,048 over 14K) 513 / 460;
+//   against it: 4.0 (eight of 512, D 64) 27.7 / 25.5, 4.7 (32 trees, 12 / 2
+//   heads) 33.9 / 33.7, 7.3 (two of 1,000) 44.4 / 43.8, 7.3 (eight of 128 over 2K,
+//   D 64) 32.9 / 31.8; 8.2 (32 trees) 56.9 / 58.3, 14.5 (512 over 8K, D 64) 38.3 /
+//   42.0, 15.9 (eight of 200 over 1,000, 32 / 8 heads) 69.1 / 70.3.
+// (At D 64 tiles per workgroup do not tell the two apart well.)
 constexpr int64_t kWideShareTiles = 8;
 
 int64_t choose_prefill_waves(const Requests& q, const PrefillParams& p, int64_t slots_per_head8, bool wide_built,

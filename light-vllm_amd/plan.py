@@ -73,7 +73,9 @@ UNIT_TOKENS = 32
 # tiles per request): 39.9 us at four tiles per wave against 47.5 us at one,
 # i.e. 4 x 39.9 / 47.5 = 3.4 per token.
 COL_TILES4_COST = 3.4
-PREFILL_WIDE_MAX_TILES = 20  # mean key tiles per unit up to which 8-wave prefill workgroups win
+# Mean key tiles per unit up to which 8-wave prefill workgroups win where units
+# may not be split (elsewhere the native planner counts tiles per workgroup).
+PREFILL_WIDE_MAX_TILES = 20
 
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
@@ -176,33 +178,6 @@ class Staging:
             offsets.append(off)
             off += n
         return self.upload(buf[:off]), offsets
-
-
-def choose_prefill_waves(
-    *, q_lens: np.ndarray, computed: np.ndarray, rows: np.ndarray, group: int, columns: int, key_tokens: int,
-    slots_per_head: int, wide_built: bool,
-) -> int:
-    """A first estimate of the prefill workgroup shape from the units' count
-    and mean length alone: 8 waves of one column tile when there are fewer
-    units than resident workgroups or they are short (mean key tiles per unit
-    at most PREFILL_WIDE_MAX_TILES), else 4 waves of two column tiles.  A
-    step's plan takes the native planner's rule, which weighs the key tiles
-    per resident workgroup where units may be split.
-    """
-
-    if not wide_built or not rows.any():
-        return 4
-    ncols = q_lens * group
-    nunit = np.where(rows, -(-ncols // columns), 0)
-    n = int(nunit.sum())
-    req = np.repeat(np.arange(len(q_lens)), nunit)
-    starts = np.zeros(len(q_lens), dtype=np.int64)
-    np.cumsum(nunit[:-1], out=starts[1:])
-    col0 = (np.arange(n) - starts[req]) * columns
-    last = np.minimum(col0 + columns, ncols[req]) - 1
-    tiles = -(-(computed[req] + last // group + 1) // key_tokens)
-    split = bool(slots_per_head) and n < slots_per_head
-    return 8 if split or float(tiles.mean()) <= PREFILL_WIDE_MAX_TILES else 4
 
 
 class DecodeWork:
@@ -491,17 +466,6 @@ class StepPlan:
             four = float((seq * -(-nct // 4)).sum()) * COL_TILES4_COST
             found = self._col_tiles[key] = 4 if four < one else 1
         return found
-
-    def prefill_waves(self, group: int, num_kv_heads: int, prefill_columns: int, prefill_key_tokens: int,
-                      prefill_resident: int, wide_built: bool) -> int:
-        """The prefill workgroup shape (4 or 8 waves) for this step's wide rows."""
-
-        rows = ~self.decode_rows(prefill_columns, group)
-        return choose_prefill_waves(
-            q_lens=self.facts.q_lens, computed=self.facts.computed, rows=rows, group=group, columns=prefill_columns,
-            key_tokens=prefill_key_tokens,
-            slots_per_head=prefill_resident // num_kv_heads if prefill_resident else 0, wide_built=wide_built,
-        )
 
     def work(
         self, group: int, num_kv_heads: int, resident_waves: int = 8 * NUM_CUS, prefill_columns: int = 0,

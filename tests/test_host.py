@@ -940,23 +940,26 @@ def test_one_call_step_plan_equals_the_per_shape_plan(seed, small_buffer, monkey
 
 
 def test_prefill_shape_choice_follows_the_measured_workloads() -> None:
-    """8-wave prefill workgroups for split-K or short units, 4-wave for long
-    unsplit units (the kernel notes hold the measurements)."""
+    """8-wave prefill workgroups for few key tiles per resident workgroup (or,
+    where units may not be split, short units), else 4-wave (the planner's
+    notes hold the measurements)."""
 
-    from light_vllm_amd.plan import choose_prefill_waves
+    def pick(q_lens, computed, group, slots_per_head=128, split=1, wide=1):
+        blocks = [-(-(c + n) // 16) for c, n in zip(computed, q_lens)]
+        md = lv.PagedAttentionMetadata(
+            block_tables=tuple(tuple(range(sum(blocks[:i]), sum(blocks[:i + 1]))) for i in range(len(blocks))),
+            num_computed_tokens=tuple(computed), query_layouts=tuple(lv.linear_query_layout(n) for n in q_lens))
+        facts = (group, 2, 16, 128, 64, split, 0, 0, 1, wide, 1024, 32, 0, 0, 2 * slots_per_head, 2 * slots_per_head,
+                 0, 16, 1, 4, 0, 0, 0, 0, 8)
+        return StepPlan(md, block_size=16, device=CPU).layer_work(facts).prefill_waves
 
-    def pick(q_lens, computed, group, slots_per_head=128, wide=True):
-        q_lens = np.asarray(q_lens, dtype=np.int64)
-        return choose_prefill_waves(q_lens=q_lens, computed=np.asarray(computed, dtype=np.int64),
-                                    rows=q_lens * group > 16, group=group, columns=128, key_tokens=64,
-                                    slots_per_head=slots_per_head, wide_built=wide)
-
-    assert pick([512] * 8, [3072] * 8, 7) == 4           # long chunks, no split
-    assert pick([512] * 8, [0] * 8, 7) == 8              # short units
+    assert pick([512] * 8, [3072] * 8, 7) == 4           # long chunks
+    assert pick([512] * 7, [0] * 7, 7) == 8              # few short units
     assert pick([9] * 32, [2300] * 32, 6, 256) == 8      # C5 tree verification: split
-    assert pick([512] * 2, [16384] * 2, 7) == 8          # few units over long history: split
-    assert pick([512] * 8, [3072] * 8, 7, 0) == 4        # splitting disabled, long units
-    assert pick([9] * 32, [2300] * 32, 6, 256, wide=False) == 4
+    assert pick([512] * 2, [16384] * 2, 7) == 4          # few units over long history: split in long pieces
+    assert pick([512] * 8, [3072] * 8, 7, split=0) == 4  # splitting disabled, long units
+    assert pick([512] * 8, [0] * 8, 7, split=0) == 8     # splitting disabled, short units
+    assert pick([9] * 32, [2300] * 32, 6, 256, wide=0) == 4
     assert pick([1] * 8, [100] * 8, 7) == 4              # no prefill rows
 
 
