@@ -987,7 +987,7 @@ struct MergeArgs {
   const float* part_ml;
   void* out;
   int64_t out_tok_stride, out_head_stride;
-  FastDiv by_group;  // / group
+  FastDiv by_group, by_cols;  // / group, / columns per partial slot
 };
 
 constexpr int kMergeRoundTrip = 16;  // partials a wave requests at once
@@ -1040,7 +1040,7 @@ __global__ __launch_bounds__(64 * merge_waves(P)) void paged_merge_kernel(
   const int span_slot = jb[6] - 1;
   const int span_pieces = span_slot >= 0 ? (int)((uint32_t)jb[7] >> 24) : 0;
   const int sv = (jb[7] & 0xffffff) + col;
-  const int sunit = sv / cols;
+  const int sunit = fast_div(sv, a.by_cols);
   const int scol = sv - sunit * cols;
   const int ntot = np + span_pieces;
   // Partial rows of this column: its own pieces, then its span unit's.
@@ -1244,7 +1244,7 @@ int launch_merge(const void* part_acc, const float* part_ml, void* out, int64_t 
   if (num_jobs < 0 || num_kv_heads <= 0 || group <= 0) return LVAMD_ERR_INVALID_ARGUMENT;
   if (num_jobs == 0) return LVAMD_OK;
   if (!part_acc || !part_ml || !out || !jobs) return LVAMD_ERR_INVALID_ARGUMENT;
-  MergeArgs a{.by_group = FastDiv(group)};
+  MergeArgs a{.by_group = FastDiv(group), .by_cols = FastDiv(16 * col_tiles)};
   a.part_acc = part_acc;
   a.part_ml = part_ml;
   a.out = out;
