@@ -202,8 +202,9 @@ constexpr int split_waves() {
 // Column c's chunk q sits at chunk slot c * D/4 + (q + c) % (D/4): the rows'
 // stride is a multiple of the 64 LDS banks for D = 64 and 128, so unrotated
 // rows put the same chunk of all 16 columns (what a wave writes, and reads
-// back) on the same four banks; rotated by the column they fall on all 64
-// (for every D: D/4 + 1 is odd).
+// back) on the same four banks; rotated by the column they fall on all 64.
+// So for D = 192 and 256; for the other head sizes the rotation wraps before
+// the banks do and two columns share theirs (four or eight do unrotated).
 template <int D>
 __device__ __forceinline__ int result_chunk(int c, int q) {
   constexpr unsigned CH = D / 4;
