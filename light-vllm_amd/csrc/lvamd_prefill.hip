@@ -17,8 +17,8 @@
 //     step's K/V) into LDS (global_load_lds_dwordx4: no registers, no LDS
 //     store instructions), double-buffered, one barrier per tile: tile t+1
 //     lands while tile t computes, tile t+2's table entries are in flight.
-//     With blocks of 16 tokens or more the 16 rows that a wave loads lie in
-//     one block, so their addresses are scalar (the B16 kernels).
+//     With block sizes that are powers of two from 16 the 16 rows that a wave
+//     loads lie in one block, so their addresses are scalar (the B16 kernels).
 //     The LDS layout is unpadded and XOR-swizzled (below) so that the
 //     loads, the K reads and the V transpose reads are all free of bank
 //     conflicts.
